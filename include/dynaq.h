@@ -347,9 +347,10 @@ typedef enum dq_kernel {
 } dq_kernel;
 
 /* DQ_KERNEL_F32_EXPAND_GEMM runs on the matrix cores from this many rows on: weight
- * tiles expanded to fp32 as the reference's x86 expansion does (one fma per value),
- * contracted with the fp32 rows on v_mfma_f32 (sums in the matrix cores' order, within
- * 1e-5 of sum |x_k w_k|; a row's outputs do not depend on the other rows). Fewer rows
+ * values as the reference's x86 expansion has them (a code times its block's scale),
+ * contracted with the fp32 rows, split exactly into three bf16 parts, on the bf16 matrix
+ * cores (sums in their order, within 1e-5 of sum |x_k w_k|; a row's outputs do not depend
+ * on the other rows). Fewer rows
  * run the fp32 row-dot GEMV, the same class in vec_dot order. */
 #define DQ_F32_GEMM_MIN_ROWS 16
 
