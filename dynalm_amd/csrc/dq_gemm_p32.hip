@@ -13,9 +13,8 @@
 // accumulator, which ends at exactly sc_j P_j 2^-24. Then
 //   per sub-block:    T = fma(da_j, sc_j P_j 2^-24, T)      (one VALU operation per output)
 //   per super-block:  acc = fma(d 2^24, T, acc)             (one per output), T = 0
-// and the mins term as fp32 matrix products on v_mfma_f32_32x32x2_f32, two
-// sub-blocks per instruction straight into the output accumulator:
-//   acc = acc + sum_j (-dmin m_j) c_j.
+// and the mins term Mn = sum_j m_j c_j on two v_mfma_f32_32x32x16_bf16 per super-block (m_j
+// < 64 is exact in bf16; c_j is the exact sum of three bf16 parts), acc = fma(-dmin, Mn, acc).
 // Every product is exact or rounded once, but d multiplies the super-block's sum
 // rather than each term, and the summation order is not qmm's (nor the per-32
 // GEMV's, kernels_generic.cpp:261-279): the outputs agree within the fp32 tolerance of
@@ -26,12 +25,17 @@
 // activation tiles. The weight rows are the MFMA's A operand (lane l builds row l % 32's
 // operand from nibbles it loads itself, each serving four MFMAs), the activation rows
 // its B operand, so a lane's 16 results share one activation row and the
-// per-sub-block activation scale da_j is one register per tile, read ahead of the
-// sub-block. K-steps 2 j and 2 j + 1 belong to sub-block j alone; after them the wave
-// folds the sub-block into T (VALU) while the SIMD's other wave runs MFMAs. A
-// super-block's operands (128 rows x 256 codes as f16, 64 KB), activation scales and
-// mins operands (4 + 4 KB) go to LDS one interval ahead by direct-to-LDS loads spread
-// over the K-steps, into a ring of two; one barrier per super-block.
+// per-sub-block activation scale da_j is one register per tile. K-steps 2 j and 2 j + 1
+// belong to sub-block j alone; each tile's result is folded into T (VALU) behind the next
+// tile's two MFMAs. A super-block's operands (128 rows x 256 codes as f16, 64 KB), activation
+// scales and mins operands (4 + 8 KB) go to LDS one interval ahead by direct-to-LDS loads
+// spread over the steps, into a ring of two; one barrier per super-block.
+// What bounds it: issue slots. A wave's super-block is 72 MFMAs and ~870 VALU (the folds 640,
+// the weight operands ~200); two waves per SIMD need 15 clocks of issue per MFMA and 4 per
+// VALU (measured in a register-only loop), 147 K clocks in all at K = 4096, ~65 us. M = 512,
+// N = 14336, kernel alone: 109 -> 96 us; the whole call 112.6 -> 102; M = 77, N = 5003, K =
+// 2304 28.8 -> 25.9. Without its loads 109 of 115 us, without the operand build 105, with a
+// quarter of the folds 99 (graph replay).
 //
 // Activation layout ("act32", k_act32_from_p32 from per-32 rows), for M_pad = m
 // rounded up to the workgroup's 32 TT rows (zero rows past m), T = M_pad / 32 row
@@ -40,7 +44,8 @@
 //          hh = l / 32; K-step k = 2 j + h holds values 32 j + 16 hh + 8 h + {0, 2, 1,
 //          3, 4, 6, 5, 7} of the super-block (sub-block j only)
 //   da     [T][nb][j (8)][32 rows] floats
-//   c      [T][nb][kk (4)][lane (64)] floats: c of row l % 32, sub-block 2 kk + l / 32
+//   c      [T][nb][part (2)][lane (64)][8 bf16]: row l % 32's eight c_j 2^-9; part 0 hi (lanes
+//          0-31) and mid, part 1 lo and zeros
 // The K order is the one in which a lane's B operand comes out of two dwords of its
 // weight row's nibbles: values 32 j + t of sub-block j are the low (j even) or high
 // (j odd) nibbles of qs bytes 32 (j / 2) + t (quant_formats.cpp:150-167), so K-step
@@ -62,18 +67,45 @@ namespace {
 constexpr int kPN = 256;  // weight rows per workgroup (activation rows: 32 TT)
 constexpr int kPThreads = 512;       // 8 waves, two per SIMD
 // Super-block buffer: operands [k (16)][t (4)][lane (64)][16 B], then the activation
-// scales [t (4)][j (8)][row (32)] and the mins operands [t (4)][kk (4)][lane (64)].
+// scales [t (4)][j (8)][row (32)] and the mins operands [t (4)][part (2)][lane (64)][16 B].
 // With TT 32-row activation tiles per workgroup (TT = 4, or 2 / 1 for few rows): codes
-// 16 TT KB, scales and mins operands TT KB each.
+// 16 TT KB, scales TT KB, mins operands 2 TT KB.
 template <int TT>
 struct PLds {
   static constexpr int kCodes = 16 * TT * 1024, kDa = kCodes, kC = kDa + TT * 1024;
-  static constexpr int kBuf = kC + TT * 1024;
-  static constexpr int kTotal = 2 * kBuf;
+  static constexpr int kBuf = kC + 2 * TT * 1024;
+  static constexpr int kRow = 2 * kBuf;  // per wave: d 2^24, then -dmin 2^9, of its 32 weight rows
+  static constexpr int kTotal = kRow + 8 * 256;
 };
 static_assert(PLds<4>::kTotal <= 160 * 1024, "LDS");
 
-DQ_DEV v16f_t mfma_f32_k2(float a, float b, v16f_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
+DQ_DEV v16f_t mfma_bf(v4u a, v4u b, v16f_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, a), __builtin_bit_cast(v8bf_t, b), c, 0, 0,
+                                                 0);
+}
+DQ_DEV u32 bf_pair(float a, float b) {
+  typedef float v2f_t __attribute__((ext_vector_type(2)));
+  typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(u32, __builtin_convertvector(v2f_t{a, b}, v2bf_t));
+}
+// c of one (row, sub-block j) into the mins operands of its tile and super-block at cb, times
+// 2^-9 so that sum_j m_j c_j (at most 504 times the largest) stays finite before dmin comes to
+// it: hi + mid + lo exactly in bf16; part 0 holds hi (lanes 0-31) and mid (32-63), part 1 lo and
+// zeros, each lane its row's eight sub-blocks.
+DQ_DEV void put_c(uint8_t* cb, int r, int j, float c) {
+  c *= 0x1p-9f;
+  // hi truncated, so that a finite c stays finite; an infinite or NaN c is hi alone
+  const u32 hi = as_u(c) & 0xFFFF0000u;
+  const float c1 = fabsf(c) <= 3.40282347e38f ? c - as_f(hi) : 0.0f;
+  const u32 mid = bf_pair(c1, 0.0f);
+  const u32 lo = bf_pair(c1 - as_f(mid << 16), 0.0f);
+  uint16_t* o = reinterpret_cast<uint16_t*>(cb + r * 16) + j;
+  o[0] = (uint16_t)(hi >> 16 | (c != c ? 1u : 0u));  // a NaN whose high bits are an infinity's
+  o[256] = (uint16_t)mid;
+  o[512] = (uint16_t)lo;
+  o[768] = 0;
+}
 
 }  // namespace
 
@@ -106,15 +138,15 @@ __global__ __launch_bounds__(256) void k_act32_from_p32(const uint8_t* __restric
     *reinterpret_cast<float*>(out + codes_bytes + (T * nb + s) * 1024 + t * 4) = d;
   }
   {
-    // c = d * (code sum): thread t = 64 kk + lane, sub-block 2 kk + lane / 32
-    const int l = t & 63, j = 2 * (t >> 6) + (l >> 5);
-    const int64_t row = 32 * T + (l & 31);
+    // c = d * (code sum): thread t = 32 j + r
+    const int j = t >> 5;
+    const int64_t row = 32 * T + (t & 31);
     float c = 0.0f;
     if (row < m) {
       const uint8_t* b = acts + row * arb + (int64_t)(8 * s + j) * 40;
       c = *reinterpret_cast<const float*>(b) * (float)*reinterpret_cast<const int32_t*>(b + 4);
     }
-    *reinterpret_cast<float*>(out + codes_bytes + da_bytes + (T * nb + s) * 1024 + t * 4) = c;
+    put_c(out + codes_bytes + da_bytes + (T * nb + s) * 2048, t & 31, j, c);
   }
 }
 
@@ -146,8 +178,7 @@ __global__ __launch_bounds__(64) void k_act32_quant(const float* __restrict__ x,
   if ((l & 7) == 0) {
     float* dab = reinterpret_cast<float*>(out + codes_bytes + (T * nb + s) * 1024);
     dab[j * 32 + r] = d;
-    float* cb = reinterpret_cast<float*>(out + codes_bytes + da_bytes + (T * nb + s) * 1024);
-    cb[(j >> 1) * 64 + 32 * (j & 1) + r] = d * (float)sum;
+    put_c(out + codes_bytes + da_bytes + (T * nb + s) * 2048, (int)r, j, d * (float)sum);
   }
 }
 
@@ -188,7 +219,7 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
   const int64_t mbase = (int64_t)tm * 32 * TT;
 
   const int64_t codes_bytes = m_pad * nb * 512, da_bytes = m_pad / 32 * nb * 1024;
-  const auto ra = rsrc(act32, (u32)(codes_bytes + 2 * da_bytes));
+  const auto ra = rsrc(act32, (u32)codes_bytes), rc = rsrc(act32 + codes_bytes, (u32)(3 * da_bytes));
   const auto rq = rsrc(qs_plane, (u32)(n_pad * nb * 128));
   const auto rh = rsrc(hdr_plane, (u32)(n_pad * nb * 16));
 
@@ -202,8 +233,8 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
   const u32 vq = (G * (u32)nb * 8u + (u32)hh) * 1024u + r64 * 16u;  // + (s * 8 + 2 g) * 1024
   const u32 vh = (G * (u32)nb * 64u + r64) * 16u;                  // + s * 1024
 
-  auto issue_piece = [&](int s, int i) {
-    uint8_t* P = lds + (s & 1) * X::kBuf;
+  auto issue_piece = [&](int s, int buf, int i) {
+    uint8_t* P = lds + buf * X::kBuf;
     const int jb = 2 * TT * wave + i;
     const int64_t T = (int64_t)TT * tm + (jb % TT);
     dma16(ra, P + jb * 1024, (u32)(lane * 16), (u32)(((T * nb + s) * 16 + (jb / TT)) * 1024));
@@ -211,9 +242,11 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
       const int tt = wave & 3;
       const int64_t Tb = (int64_t)TT * tm + tt;
       if (wave < TT) {
-        dma16(ra, P + X::kDa + tt * 1024, (u32)(lane * 16), (u32)(codes_bytes + (Tb * nb + s) * 1024));
+        dma16(rc, P + X::kDa + tt * 1024, (u32)(lane * 16), (u32)((Tb * nb + s) * 1024));
       } else if (wave >= 4 && wave < 4 + TT) {
-        dma16(ra, P + X::kC + tt * 1024, (u32)(lane * 16), (u32)(codes_bytes + da_bytes + (Tb * nb + s) * 1024));
+        const u32 o = (u32)(da_bytes + (Tb * nb + s) * 2048);
+        dma16(rc, P + X::kC + tt * 2048, (u32)(lane * 16), o);
+        dma16(rc, P + X::kC + tt * 2048 + 1024, (u32)(lane * 16), o + 1024);
       }
     }
   };
@@ -224,117 +257,155 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
   v4u nib[4], hdr, hdr_n;
   auto ld_nib = [&](int s, int g) { return ld16(rq, vq + (u32)((s < nb ? s : nb - 1) * 8 + 2 * g) * 1024u); };
   auto ld_hdr = [&](int s) { return ld16(rh, vh + (u32)(s < nb ? s : nb - 1) * 1024u); };
+  // The lane's weight row (get_scale_min_k4, quant_formats.h:62-70): sc_j bytes of sub-blocks
+  // 0..3 and 4..7.
+  auto scales = [](v4u h, u32& a, u32& b) {
+    a = h.y & 0x3F3F3F3Fu;
+    b = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
+  };
+  // weight operand of K-step k = 2 j + h: sc_j times 8 nibbles of two dwords, in the pair
+  // order
+  auto build = [&](int k, u32 scA, u32 scB) -> v4u {
+    const int j = k >> 1, h = k & 1;
+    u32 x0 = nib[j >> 1][2 * h], x1 = nib[j >> 1][2 * h + 1];
+    const u32 sp = __builtin_amdgcn_perm(0u, j < 4 ? scA : scB, sel_u16x2(j & 3));
+    v4u w;
+    if (j & 1) {
+      auto hi = [&](u32 x, int sh) { return mul_bytes(((x >> sh) & 0x000F000Fu) ^ 0x00080008u, sp); };  // the plane's XOR 8
+      w = v4u{hi(x0, 4), hi(x0, 12), hi(x1, 4), hi(x1, 12)};
+    } else {
+      w = v4u{mul_bytes(x0 & 0x000F000Fu, sp), mul_bytes((x0 >> 8) & 0x000F000Fu, sp),
+              mul_bytes(x1 & 0x000F000Fu, sp), mul_bytes((x1 >> 8) & 0x000F000Fu, sp)};
+    }
+    asm volatile("" : "+v"(w));  // built here, not beside its first MFMA
+    return w;
+  };
 
-  v16f_t acc[TT], S[TT], T[TT];
+  v16f_t acc[TT], T[TT];
 #pragma unroll
-  for (int mt = 0; mt < TT; ++mt) {
-    acc[mt] = v16f_t{};
-    S[mt] = v16f_t{};
-  }
+  for (int mt = 0; mt < TT; ++mt) acc[mt] = v16f_t{};
+  v4u w[2];  // the two K-steps' weight operands of the coming sub-block
+  uint8_t* const rowd = lds + X::kRow + wave * 256;
 
-  // Super-block s: per sub-block j its two K-steps (TT MFMA chains, one per activation
-  // tile) and then its fold into T; the next super-block's loads spread over the K-steps,
-  // and the 4 TT mins products over the even K-steps; at the end T into acc.
+  // Super-block s in 9 TT steps of two MFMAs, one (sub-block j, tile tt) each, then the mins of
+  // each tile as j = 8. A step folds the step before's result while its own MFMAs run, reads
+  // the next step's operands and does its share of the rest (the next sub-block's weight
+  // operands, the next super-block's loads). A wave issues in order, so the fences put half of
+  // a step's VALU behind each MFMA; with all of a sub-block's MFMAs in one run and its folds
+  // after them the kernel took 109 us at M = 512 (K = 4096, N = 14336), now 96.
   auto run_sb = [&](int s) {
-    const bool next = s + 1 < sb1;
+    const int sn = s + 1 < nb ? s + 1 : nb - 1;
     hdr_n = ld_hdr(s + 1);
     const uint8_t* P = lds + __builtin_amdgcn_readfirstlane((s & 1) * X::kBuf);
-    // this lane's weight row (get_scale_min_k4, quant_formats.h:62-70): sc_j as (sc, sc)
-    // 16-bit pairs, m_j, d and dmin
-    const u32 scA = hdr.y & 0x3F3F3F3Fu;
-    const u32 scB = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
-    const u32 mA = hdr.z & 0x3F3F3F3Fu;
-    const u32 mB = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
-    const float ndm = -h2f(hdr.x >> 16);
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) T[tt] = v16f_t{};
-    // mins product kk of tile tt: A = -dmin m_j of this lane's row, B = c of the lane's
-    // activation row, K index hh: sub-block 2 kk + hh
-    auto mins = [&](int tt, int kk) {
-      const int j = 2 * kk + hh;
-      const float am = ndm * (float)((j < 4 ? mA : mB) >> (8 * (j & 3)) & 0xFFu);
-      const float cv = as_f(lds4v(P + X::kC + ((tt * 4 + kk) * 64 + lane) * 4));
-      acc[tt] = mfma_f32_k2(am, cv, acc[tt]);
-    };
-    // weight operand of K-step k = 2 j + h: sc_j times 8 nibbles of two dwords, in the
-    // pair order
-    auto build = [&](int k) -> v4u {
-      const int j = k >> 1, h = k & 1;
-      u32 x0 = nib[j >> 1][2 * h], x1 = nib[j >> 1][2 * h + 1];
-      asm volatile("" : "+v"(x0), "+v"(x1));  // keeps this K-step's operand build here
-      const u32 sp = __builtin_amdgcn_perm(0u, j < 4 ? scA : scB, sel_u16x2(j & 3));
-      if (j & 1) {
-        x0 ^= 0x80808080u;  // the plane's high nibbles XOR 8, undone
-        x1 ^= 0x80808080u;
-        return v4u{mul_bytes((x0 >> 4) & 0x000F000Fu, sp), mul_bytes((x0 >> 12) & 0x000F000Fu, sp),
-                   mul_bytes((x1 >> 4) & 0x000F000Fu, sp), mul_bytes((x1 >> 12) & 0x000F000Fu, sp)};
+    u32 scA, scB;
+    scales(hdr, scA, scB);
+    v4u a0, a1;
+    float da = 0;
+    auto rd = [&](int j, int tt) {  // the operands of step (j, tt)
+      if (j < 8) {
+        a0 = lds16(P + ((TT * 2 * j + tt) * 64 + lane) * 16);
+        a1 = lds16(P + ((TT * (2 * j + 1) + tt) * 64 + lane) * 16);
+        da = *reinterpret_cast<const float*>(P + X::kDa + ((tt * 8 + j) * 32 + li) * 4);
+      } else {
+        a0 = lds16(P + X::kC + tt * 2048 + lane * 16);
+        a1 = lds16(P + X::kC + tt * 2048 + 1024 + lane * 16);
       }
-      return v4u{mul_bytes(x0 & 0x000F000Fu, sp), mul_bytes((x0 >> 8) & 0x000F000Fu, sp),
-                 mul_bytes(x1 & 0x000F000Fu, sp), mul_bytes((x1 >> 8) & 0x000F000Fu, sp)};
     };
-    // da_j of this lane's activation row in tile tt
-    auto ld_da = [&](int tt, int j) { return as_f(lds4v(P + X::kDa + ((tt * 8 + j) * 32 + li) * 4)); };
-    float da[TT];
-    v4u w = build(0);
+    rd(0, 0);
+    v16f_t sp{};
+    float dp = 0;
+    v4u mm{};
+    // the result of step (j, tt): T += da_j sc_j P_j; the mins and then the super-block's sum
+    // into acc with -dmin 2^9 and d 2^24 of the lane's 16 weight rows 8 q + 4 hh + e
+    auto fold = [&](int j, int tt) {
+      if (j < 8) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      __builtin_amdgcn_s_setprio(2);
-      if ((k & 1) == 0) {
-        // the sub-block's activation scales, used after its two K-steps; the super-block's
-        // mins products q = tile 4 + pair, 4 TT of them over the 8 even K-steps (TT = 4:
-        // two per even K-step; 2: one; 1: one every other)
+        for (int r = 0; r < 16; ++r) T[tt][r] = j == 0 ? dp * sp[r] : fmaf(dp, sp[r], T[tt][r]);
+        asm volatile("" : "+v"(T[tt]));
+      } else {
 #pragma unroll
-        for (int tt = 0; tt < TT; ++tt) da[tt] = ld_da(tt, k >> 1);
-        if (TT == 4) {
-          mins(k >> 2, 2 * ((k >> 1) & 1));
-          mins(k >> 2, 2 * ((k >> 1) & 1) + 1);
-        } else if (TT == 2) {
-          mins((k >> 1) >> 2, (k >> 1) & 3);
-        } else if ((k & 3) == 0) {
-          mins(0, k >> 2);
+        for (int q = 0; q < 4; ++q) {
+          const v4u d = lds16(rowd + (8 * q + 4 * hh) * 4), nd = lds16(rowd + 128 + (8 * q + 4 * hh) * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int r = 4 * q + e;
+            acc[tt][r] = fmaf(as_f(d[e]), T[tt][r], fmaf(as_f(nd[e]), sp[r], acc[tt][r]));
+          }
+        }
+        asm volatile("" : "+v"(acc[tt]));
+      }
+    };
+#pragma unroll
+    for (int q = 0; q < 9 * TT; ++q) {
+      const int j = q / TT, tt = q % TT;
+      const v4u b0 = a0, b1 = a1;
+      const float db = da;
+      if (q + 1 < 9 * TT) rd((q + 1) / TT, (q + 1) % TT);
+      v16f_t S;
+      v4u wn[2];
+      if (j < 8) {
+        S = mfma_h(w[0], b0, v16f_t{});
+        S = mfma_h(w[1], b1, S);
+      } else {
+        S = mfma_bf(mm, b0, v16f_t{});
+        S = mfma_bf(mm, b1, S);
+      }
+      if (q > 0) fold((q - 1) / TT, (q - 1) % TT);
+      // the next sub-block's weight operands (j = 8: the next super-block's first), nib[g] and
+      // its reload once its last operand is built
+      u32 sA = scA, sB = scB;
+      if (j == 8) scales(hdr_n, sA, sB);
+      if (j != 7) {
+        const int k = 2 * (j == 8 ? 0 : j + 1);
+        if (tt == (TT - 1) / 2) wn[0] = build(k, sA, sB);
+        if (tt == TT - 1) {
+          wn[1] = build(k + 1, sA, sB);
+          if (k > 0 && (k & 2)) nib[k >> 2] = ld_nib(s + 1, k >> 2);
         }
       }
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) {
-        const v4u a = lds16(P + ((TT * k + tt) * 64 + lane) * 16);
-        S[tt] = mfma_h(w, a, (k & 1) == 0 ? v16f_t{} : S[tt]);
+      if (q == 4 * TT) {  // d 2^24 and -dmin 2^9 of the wave's weight rows (both lane halves alike)
+        *reinterpret_cast<float*>(rowd + li * 4) = h2f(hdr.x) * 16777216.0f;
+        *reinterpret_cast<float*>(rowd + 128 + li * 4) = h2f(hdr.x >> 16) * -512.0f;
       }
-      if (k < 15) w = build(k + 1);
-      // the next super-block's 2 TT pieces of this wave, evenly over the K-steps
-      if (k % (8 / TT) == 0 && next) issue_piece(s + 1, k / (8 / TT));
-      if ((k & 3) == 3) nib[k >> 2] = ld_nib(s + 1, k >> 2);
+      if (j == 7 && tt == TT - 1) {  // the mins' weight operand: m_j of the lane's row
+        const u32 mA = hdr.z & 0x3F3F3F3Fu, mB = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
+        auto mf = [](u32 v, int i) { return (float)((v >> (8 * i)) & 0xFFu); };
+        mm = v4u{bf_pair(mf(mA, 0), mf(mA, 1)), bf_pair(mf(mA, 2), mf(mA, 3)), bf_pair(mf(mB, 0), mf(mB, 1)),
+                 bf_pair(mf(mB, 2), mf(mB, 3))};
+      }
+      // the next super-block's 2 TT pieces of this wave, one every fourth step (past the end the
+      // last one's again, into the buffer no one reads)
+      if (q % 4 == 1 && q / 4 < 2 * TT) issue_piece(sn, (s + 1) & 1, q / 4);
+      __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+      }
+      sp = S;
+      dp = db;
+      if (tt == TT - 1 && j != 7) {
+        w[0] = wn[0];
+        w[1] = wn[1];
+      }
       __builtin_amdgcn_sched_barrier(0);
-      if (k & 1) {
-        // sub-block j = k / 2 done: T += da_j sc_j P_j over the tiles
-        __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-        for (int tt = 0; tt < TT; ++tt) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) T[tt][r] = fmaf(da[tt], S[tt][r], T[tt][r]);
-          asm volatile("" : "+v"(T[tt]));  // the sub-block's results exist here, not after later MFMAs
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
     }
-    // acc += d 2^24 T: d of the lane's 16 result rows 8 (r / 4) + 4 hh + r % 4, which lanes
-    // 0-31 hold (one weight row each)
-    const float d24 = h2f(hdr.x) * 16777216.0f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int src = 8 * (r >> 2) + 4 * hh + (r & 3);
-      const float dr = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * src, __builtin_bit_cast(int, d24)));
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) acc[tt][r] = fmaf(dr, T[tt][r], acc[tt][r]);
-    }
+    fold(8, TT - 1);
   };
 
   // prologue: the first super-block's operands and weights
 #pragma unroll
-  for (int i = 0; i < 2 * TT; ++i) issue_piece(sb0, i);
+  for (int i = 0; i < 2 * TT; ++i) issue_piece(sb0, sb0 & 1, i);
   hdr = ld_hdr(sb0);
 #pragma unroll
   for (int g = 0; g < 4; ++g) nib[g] = ld_nib(sb0, g);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  {
+    u32 scA, scB;
+    scales(hdr, scA, scB);
+    w[0] = build(0, scA, scB);
+    w[1] = build(1, scA, scB);
+  }
   lds_barrier();
 #pragma unroll 1
   for (int s = sb0; s < sb1; ++s) {
@@ -389,15 +460,16 @@ int64_t act32_rows(int64_t m) {
 
 int64_t act32_bytes(int64_t m, int64_t k) {
   const int64_t mp = act32_rows(m), nb = k / 256;
-  return mp * nb * 512 + 2 * (mp / 32) * nb * 1024;
+  return mp * nb * 512 + 3 * (mp / 32) * nb * 1024;
 }
 
 bool gemm_p32_ok(const WeightDev& w, int64_t m, int64_t n0, int64_t n1) {
   if (w.dtype != kQ4_K || m <= 0 || n1 <= n0 || w.nblk <= 0) return false;
-  // 32-bit buffer offsets: the qs plane plus one tile's rows past its end, and act32;
+  // 32-bit buffer offsets: the qs plane plus one tile's rows past its end, and act32's codes
+  // (with its scales: the rows taken before the mins operands grew);
   // the writer's grid has one row of workgroups per 32 padded rows
   if ((w.n_pad + 4 * kRowGroup) * w.nblk * 128 >= (1ll << 32)) return false;
-  if (act32_bytes(m, w.k) >= (1ll << 32) || act32_rows(m) / 32 > 65535) return false;
+  if (act32_rows(m) * w.nblk * 576 >= (1ll << 32) || act32_rows(m) / 32 > 65535) return false;
   return true;
 }
 
