@@ -175,6 +175,20 @@ int with_stream_ws(int device, void* stream, size_t need, F&& fn) {
   return fn(static_cast<uint8_t*>(e->p));
 }
 
+// Whether with_stream_ws can serve `need` bytes now: the stream's workspace holds them or may
+// grow, which a stream under capture may not.
+bool stream_ws_ready(int device, void* stream, size_t need) {
+  {
+    std::lock_guard<std::mutex> lock(g_sws_mu);
+    for (const StreamWs& x : g_sws)
+      if (x.device == device && x.stream == stream && x.bytes >= need) return true;
+  }
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(as_stream(stream), &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // not this call's error: the launches after it report their own
+  return false;
+}
+
 // The quantized-activation buffer of one matmul: the start of the caller's region,
 // or the per-device pool.
 int acts_buffer(int device, size_t need, const dq::Region& r, void** out) {
@@ -290,11 +304,9 @@ int check_out(const dq_weight* w, int64_t m, int64_t n0, int64_t n1, float* y, i
 // DQ_GEMV_MAX_ROWS for Q4_K x Q8_K, except up to 48 rows of weights with at most 4096
 // rows where the skinny GEMV's LDS holds the row (its 64-row tiles beat the GEMM's few
 // workgroups there: 9.4-11.1 vs 11.8-12.2 us at K = N = 4096, 19.0-20.3 vs 22.7-23.1 at
-// K = 8960, N = 1536; at N = 14336 the GEMM wins, 16.1 vs 25.2 us at 17 rows); from 13 rows for the 32-value block GEMM (Q8_0 /
-// Q4_0 x per-32; dq_matmul measured at K = 4096, N = 4096 / 14336, quantization
-// included: GEMV passes 27.9 / 30.9 us at 12 rows, 35.7 / 36.6 at 13, 41.5 / 43.8 at
-// 18; quantize + GEMM 26.9 / 32.7 at 13, 27.0 / 32.4 at 18; at K = 14336 the two are
-// equal at 13 rows, 81.7 vs 82.8 us); Q6_K x Q8_K above 64 rows, and above
+// K = 8960, N = 1536; at N = 14336 the GEMM wins, 16.1 vs 25.2 us at 17 rows); from 13 rows for
+// the 32-value block GEMM (Q8_0 / Q4_0 x per-32, the reference's block order bit for bit;
+// below that the GEMVs, rows32_pays); Q6_K x Q8_K above 64 rows, and above
 // 16 where the skinny GEMV's LDS does not hold the row's super-blocks (K = 14336:
 // 110 us against 171-611 us for the VALU GEMV's passes at 17..64 rows; but see
 // skinny_passes16) or the weight has 4096 rows or more (the
@@ -497,6 +509,22 @@ int matmul_impl(const dq_weight* w, const float* x, int64_t m, int64_t x_stride,
     if (int rc = acts_buffer(w->dev.device, (size_t)(m * arb), r, &acts); rc != DQ_OK) return rc;
     if (int rc = dq_act_quantize(fmt, x, m, w->dev.k, x_stride, acts, stream); rc != DQ_OK) return rc;
     return dq_gemv(w, fmt, acts, m, 0, w->dev.n, y, y_stride, bias, stream);
+  }
+  if (rows32_pays(w->dev, fmt, m) && !use_gemm(w->dev, fmt, m)) {
+    // Q8_0 / Q4_0 decode batches: quantize once, then the MFMA GEMV. The rows go to the
+    // region or this stream's workspace; where there is no room and none can be allocated (a
+    // stream under capture), the routes below
+    const int64_t need = m * arb;
+    auto run = [&](uint8_t* p) -> int {
+      DQ_HIP(launch_quantize(fmt, x, m, w->dev.k, m > 1 ? x_stride : w->dev.k, p, arb, s), "quantize launch");
+      DQ_HIP(launch_gemv(w->dev, fmt, p, arb, m, 0, w->dev.n, y, y_stride, bias, nullptr, s), "gemv launch");
+      return DQ_OK;
+    };
+    if (r.base != nullptr) {
+      if ((size_t)need <= r.bytes) return run(r.base);
+    } else if (need < ((int64_t)1 << 32) && m <= 65535 && stream_ws_ready(w->dev.device, stream, (size_t)need)) {
+      return with_stream_ws(w->dev.device, stream, (size_t)need, run);
+    }
   }
   if (!use_gemm(w->dev, fmt, m)) {
     // decode: quantization fused into the GEMV (one launch per pass of up to 8 rows);

@@ -1461,10 +1461,19 @@ static hipError_t gemv_rows(const WeightDev& w, int af, const uint8_t* acts, int
                             const Workspace* ws, hipStream_t s) {
   const int paf = x != nullptr && af < 0 ? (w.dtype == kQ4_K || w.dtype == kQ6_K ? kActQ8_K : kActPer32) : af;
   // rows per pass: 8, 4, 2 or 1, the most whose staged activations fit the LDS
+  const bool rows32 = dbg == nullptr && x == nullptr && rows32_pays(w, paf, m);
   int pmax = 8;
   while (pmax > 1 && gemv_lds_bytes(w.dtype, paf, pmax, 16, w.nblk, false) > kGemvMaxLds) pmax /= 2;
   for (int64_t r0 = 0; r0 < m;) {
     const int64_t left = m - r0;
+    if (rows32) {
+      // Q8_0 / Q4_0 x per-32: the MFMA GEMV in passes of up to 16 rows
+      const int64_t n = left < kRows32Max ? left : kRows32Max;
+      const hipError_t e = launch_rows32(w, acts + r0 * arb, arb, n, n0, n1, y + r0 * ys, ys, bias, s);
+      if (e != hipSuccess) return e;
+      r0 += n;
+      continue;
+    }
     const int cap = pmax < 4 ? pmax : 4;
     const int rows = left >= 8 && pmax >= 8 ? 8 : (int)(left < cap ? left : cap);
     const uint8_t* a = acts ? acts + r0 * arb : nullptr;

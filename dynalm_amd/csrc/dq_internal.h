@@ -170,6 +170,14 @@ constexpr int64_t kF32GemmMinRows = DQ_F32_GEMM_MIN_ROWS;
 hipError_t launch_gemm_b32(const WeightDev& w, int af, const uint8_t* acts, int64_t arb, int64_t m, int64_t n0,
                            int64_t n1, float* y, int64_t ys, const float* bias, hipStream_t s);
 bool gemm_b32_supported(int dtype, int af);
+// The MFMA GEMV of Q8_0 / Q4_0 weights x per-32 ActBlockQ8 rows (arb bytes apart) for up to
+// kRows32Max rows (dq_rows32.hip). No workspace.
+constexpr int64_t kRows32Max = 16;
+// Whether m rows of w (activation format af) run faster there, in passes of 16, than in the
+// VALU GEMV's passes.
+bool rows32_pays(const WeightDev& w, int af, int64_t m);
+hipError_t launch_rows32(const WeightDev& w, const uint8_t* acts, int64_t arb, int64_t m, int64_t n0, int64_t n1,
+                         float* y, int64_t ys, const float* bias, hipStream_t s);
 // Skinny MFMA GEMV on pre-quantized rows: Q4_K / Q6_K x Q8_K for 2 <= m <=
 // kSkinnyMaxRows, and x sub-scaled (DQ_ACT_SX) for 2 <= m <= kSkinnySxMaxRows;
 // hipErrorInvalidValue otherwise. ws (may be null): room for the t-terms of the split

@@ -1,0 +1,223 @@
+// dq_rows32.hip -- the decode-batch GEMV of the 32-value weight types for gfx950: Q8_0 / Q4_0
+// weights x per-32 activations for 2..16 activation rows per pass, on int8 MFMA.
+//
+// Arithmetic per output and 32-value block b (kernels_generic.cpp:210-239): P_b, the exact
+// integer dot of the codes (Q4_0: nibble - 8), t = dw_b da_b rounded to fp32, acc = fma(t,
+// (float)P_b, acc) over the blocks of a wave's slice in order, the slices added in order. The
+// slices depend on K only, so an output's bits depend neither on the row range nor on m.
+//
+// MFMA mapping (v_mfma_i32_16x16x64_i8: lane l supplies row / column l % 16 and 16 K values of
+// lane group l / 16; result lane l holds column l % 16, rows 4 (l / 16) .. + 3). A step takes
+// four blocks, lane group g holding block 4 q + g: a lane's 16 bytes of weights are then one
+// whole load (Q8_0: two) of its row, with no exchange between lanes, and a lane's activation
+// operand is a whole block of its activation row. Block g's dot is the MFMA with the
+// activation operand zeroed outside group g (eight `and`s a block, shared by the step's TC
+// weight tiles); t = dw da of all 16 x 16 outputs is one v_mfma_f32_16x16x4_f32 on the scales
+// masked alike (one product per output, rounded once); Q4_0's -8 sum(a) is the same MFMA
+// against a constant -8, once per block, as the accumulator the tiles start from. That leaves 8
+// VALU per block and tile (convert, fma) and Q4_0's 12 to split nibbles.
+//
+// The activations come quantized (one launch for the call): quantizing a lane's own block in
+// here, 32 values at ~8 VALU each in every workgroup, took 19.6 us a call against 15.
+//
+// Work split: a workgroup owns 16 TC weight rows and all of K, its W waves contiguous slices;
+// TC = 4 (the weight load instructions read 1 KB runs, the activations are prepared once per
+// 64 weight rows) while those workgroups fill the CUs, else 2 or 1.
+// What bounds it: Q4_0 K = 4096, N = 14336 at 8 rows takes 13 us for 33 MB (2.5 TB/s; before,
+// the VALU GEMV's dots of every row: 17.6). A wave's step is 48 MFMAs (~770 clocks) and ~236 VALU
+// (~940), so a workgroup's two waves per SIMD compute for ~4 us of it; two or one row of loads
+// in flight and 8 or 16 waves measured alike.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "dq_device.h"
+#include "dq_internal.h"
+#include "dq_mfma.h"
+#include "dq_quant.h"
+
+namespace dq {
+
+namespace {
+
+typedef float v4f_t __attribute__((ext_vector_type(4)));
+typedef float v16f_t __attribute__((ext_vector_type(16)));
+typedef u32 v4ua __attribute__((ext_vector_type(4), aligned(4)));  // loads of 4-byte aligned rows
+constexpr u32 kNoLoad = 0xFFFFFFF0u;  // a buffer offset past every resource: the load returns zeros
+
+// One lane's activation block: codes of values 0..15 and 16..31, the scale.
+struct ActBlk {
+  v4u lo, hi;
+  float d;
+};
+
+struct ActRaw {  // ActBlockQ8 {float d; int32 sum; int8 q[32]}
+  v4u q[2];
+  float d;
+  DQ_DEV void load(const uint8_t* row, int b) {
+    const uint8_t* p = row + (int64_t)b * 40;
+    d = *reinterpret_cast<const float*>(p);
+    q[0] = *reinterpret_cast<const v4ua*>(p + 8);
+    q[1] = *reinterpret_cast<const v4ua*>(p + 24);
+  }
+  DQ_DEV ActBlk block() const { return ActBlk{q[0], q[1], d}; }
+};
+
+// A lane's weights of one step and tile.
+template <int WT>
+struct WBlk {
+  v4u q[WT == kQ8_0 ? 2 : 1];
+  u32 d;
+  DQ_DEV void load(__amdgpu_buffer_rsrc_t rq, __amdgpu_buffer_rsrc_t rd, u32 gb, u32 r, int b, int nblk) {
+    const u32 blk = gb + (u32)b;
+    const bool in = b < nblk;
+    if constexpr (WT == kQ8_0) {
+      q[0] = ld16nt(rq, in ? (blk * 2 * 64 + r) * 16 : kNoLoad);
+      q[1] = ld16nt(rq, in ? ((blk * 2 + 1) * 64 + r) * 16 : kNoLoad);
+    } else {
+      q[0] = ld16nt(rq, in ? (blk * 64 + r) * 16 : kNoLoad);
+    }
+    d = ld2nt(rd, in ? (blk * 64 + r) * 2 : kNoLoad);
+  }
+  DQ_DEV v4u lo() const { return WT == kQ8_0 ? q[0] : q[0] & 0x0F0F0F0Fu; }
+  DQ_DEV v4u hi() const { return WT == kQ8_0 ? q[WT == kQ8_0 ? 1 : 0] : (q[0] >> 4) & 0x0F0F0F0Fu; }
+};
+
+}  // namespace
+
+// Workgroup i: weight rows [16 (t0 + i TC), + 16 TC); acts: m <= 16 rows (fp32 or ActBlockQ8)
+// `stride` bytes apart.
+template <int WT, int TC, int W>
+__global__ __launch_bounds__(64 * W) void k_rows32(const uint8_t* __restrict__ p0, const uint8_t* __restrict__ p1,
+                                                   int nblk, int64_t n_pad, int64_t t0, int64_t n0, int64_t n1,
+                                                   const uint8_t* __restrict__ acts, int64_t stride, int m,
+                                                   float* __restrict__ y, int64_t ys, const float* __restrict__ bias) {
+  extern __shared__ __align__(16) float red[];
+  const int t = threadIdx.x, lane = t & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int64_t tile0 = t0 + (int64_t)blockIdx.x * TC;
+  const auto rq = rsrc(p0, (u32)(n_pad * nblk * plane_unit(WT, 0)));
+  const auto rd = rsrc(p1, (u32)(n_pad * nblk * 2));
+  u32 gb[TC], r[TC];
+#pragma unroll
+  for (int i = 0; i < TC; ++i) {
+    const int64_t n = 16 * (tile0 + i) + c;
+    gb[i] = (u32)((n >> 6) * nblk);
+    r[i] = (u32)(n & 63);
+  }
+  // rows past m repeat the last one (their outputs are not stored); blocks past K too (their
+  // weights are zero)
+  const uint8_t* row = acts + (int64_t)(c < m ? c : m - 1) * stride;
+  auto ablk = [&](int q) { return 4 * q + g < nblk ? 4 * q + g : nblk - 1; };
+
+  const int nq = (nblk + 3) / 4, q0 = wave * nq / W, q1 = (wave + 1) * nq / W;
+  v4f_t acc[TC];
+#pragma unroll
+  for (int i = 0; i < TC; ++i) acc[i] = v4f_t{};
+  // two steps' loads in flight, quad q in set (q - q0) % 2
+  WBlk<WT> w[2][TC];
+  ActRaw a[2];
+  auto load = [&](int q, int set) {
+    a[set].load(row, ablk(q));
+#pragma unroll
+    for (int i = 0; i < TC; ++i) w[set][i].load(rq, rd, gb[i], r[i], 4 * q + g, nblk);
+  };
+  if (q0 < q1) load(q0, 0);
+  if (q0 + 1 < q1) load(q0 + 1, 1);
+  auto step = [&](int q, int set) {
+    const ActBlk x = a[set].block();
+    v4u lo[TC], hi[TC];
+    float dw[TC];
+#pragma unroll
+    for (int i = 0; i < TC; ++i) {
+      lo[i] = w[set][i].lo();
+      hi[i] = w[set][i].hi();
+      dw[i] = h2f(w[set][i].d);
+    }
+    if (q + 2 < q1) load(q + 2, set);
+    // t = dw da of the four blocks' 16 x 16 outputs: [block][4 rows]
+    v16f_t sc[TC];
+#pragma unroll
+    for (int i = 0; i < TC; ++i) sc[i] = __builtin_amdgcn_mfma_f32_16x16x1f32(x.d, dw[i], v16f_t{}, 0, 0, 0);
+#pragma unroll
+    for (int gg = 0; gg < 4; ++gg) {
+      const u32 mask = g == gg ? 0xFFFFFFFFu : 0u;
+      const v4u al = x.lo & mask, ah = x.hi & mask;
+      v4i_t c0 = {};
+      if constexpr (WT == kQ4_0) {
+        const v4u m8 = {0xF8F8F8F8u, 0xF8F8F8F8u, 0xF8F8F8F8u, 0xF8F8F8F8u};
+        c0 = mfma(ah, m8, mfma(al, m8, c0));
+      }
+#pragma unroll
+      for (int i = 0; i < TC; ++i) {
+        const v4i_t P = mfma(ah, hi[i], mfma(al, lo[i], c0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] = fmaf(sc[i][4 * gg + e], (float)P[e], acc[i][e]);
+      }
+    }
+  };
+#pragma unroll 1
+  for (int q = q0; q < q1; q += 2) {
+    step(q, 0);
+    if (q + 1 < q1) step(q + 1, 1);
+  }
+
+  // the waves' sums in wave order: element (tile i, lane, e) of wave v at ((v TC + i) 64 + lane) 4 + e
+#pragma unroll
+  for (int i = 0; i < TC; ++i) *reinterpret_cast<v4f_t*>(red + ((wave * TC + i) * 64 + lane) * 4) = acc[i];
+  __syncthreads();
+  for (int e = t; e < TC * 256; e += 64 * W) {
+    const int l = (e >> 2) & 63, mr = 4 * (l >> 4) + (e & 3);
+    const int64_t n = 16 * (tile0 + (e >> 8)) + (l & 15);
+    float v = red[e];
+#pragma unroll
+    for (int k = 1; k < W; ++k) v += red[k * TC * 256 + e];
+    if (mr < m && n >= n0 && n < n1) y[mr * ys + n] = bias ? v + bias[n] : v;
+  }
+}
+
+namespace {
+
+template <int WT, int TC, int W>
+hipError_t launch1(const WeightDev& w, const uint8_t* acts, int64_t stride, int64_t m, int64_t n0, int64_t n1, float* y,
+                   int64_t ys, const float* bias, hipStream_t s) {
+  const int64_t t0 = n0 / 16, wgs = ((n1 + 15) / 16 - t0 + TC - 1) / TC;
+  hipLaunchKernelGGL((k_rows32<WT, TC, W>), dim3((unsigned)wgs), dim3(64 * W), W * TC * 1024, s, w.plane[0],
+                     w.plane[1], (int)w.nblk, w.n_pad, t0, n0, n1, acts, stride, (int)m, y, ys, bias);
+  return hipGetLastError();
+}
+
+template <int WT>
+hipError_t launch_type(const WeightDev& w, const uint8_t* acts, int64_t stride, int64_t m, int64_t n0, int64_t n1,
+                       float* y, int64_t ys, const float* bias, hipStream_t s) {
+  const int64_t tiles = w.n_pad / 16, cus = w.cus > 0 ? w.cus : 256;
+  if (tiles >= 3 * cus) return launch1<WT, 4, 8>(w, acts, stride, m, n0, n1, y, ys, bias, s);
+  if (2 * tiles >= 3 * cus) return launch1<WT, 2, 8>(w, acts, stride, m, n0, n1, y, ys, bias, s);
+  return launch1<WT, 1, 8>(w, acts, stride, m, n0, n1, y, ys, bias, s);
+}
+
+}  // namespace
+
+// Against the VALU GEMV's passes of up to 8 rows (quantize + this kernel / fused VALU GEMV), us,
+// K = 4096 unless said: N = 14336 (64-row workgroups) Q4_0 at 4 / 5 / 8 / 12 rows 14.3 / 14.5 /
+// 14.9 / 14.8 against 12.8 / 20.4 / 20.0 / 30.6, Q8_0 18.3 / 18.5 / 18.8 / 19.2 against 15.4 /
+// 27.3 / 20.4 / 34.0; N = 4096 at 2 / 3 / 8 / 12 rows Q4_0 8.3 / 8.3 / 8.8 / 9.2 against 7.8 /
+// 9.5 / 18.0 / 28.2, Q8_0 8.4 / 8.5 / 9.5 / 10.2 against 9.4 / 10.4 / 17.2 / 27.9; N = 4096, K =
+// 14336 at 3 / 8 / 12 rows Q8_0 18.3 / 20.6 / 23.1 against 22.3 / 49.5 / 73.1. (From 13 rows the
+// calls that may take the block GEMM do: it gives the reference's block order bit for bit.)
+bool rows32_pays(const WeightDev& w, int af, int64_t m) {
+  if ((w.dtype != kQ8_0 && w.dtype != kQ4_0) || af != kActPer32 ||
+      w.n_pad * w.nblk * plane_unit(w.dtype, 0) >= (int64_t)kNoLoad) {
+    return false;
+  }
+  const bool wide = w.n_pad / 16 >= 3 * (w.cus > 0 ? w.cus : 256);
+  return m >= (wide ? 5 : 3);
+}
+
+hipError_t launch_rows32(const WeightDev& w, const uint8_t* acts, int64_t arb, int64_t m, int64_t n0, int64_t n1,
+                         float* y, int64_t ys, const float* bias, hipStream_t s) {
+  if ((w.dtype != kQ8_0 && w.dtype != kQ4_0) || m < 1 || m > kRows32Max || n1 <= n0) return hipErrorInvalidValue;
+  return w.dtype == kQ8_0 ? launch_type<kQ8_0>(w, acts, arb, m, n0, n1, y, ys, bias, s)
+                          : launch_type<kQ4_0>(w, acts, arb, m, n0, n1, y, ys, bias, s);
+}
+
+}  // namespace dq

@@ -205,7 +205,7 @@ DQ_API int dq_qmm_gemm(const dq_weight* w, int64_t n0, int64_t n1, const dq_qmm_
  * for r < m and i in [n0, n1). `acts`: m rows in format fmt, as dq_act_quantize
  * writes them. Replaces qmm::Kernels::gemv (dynacore/include/dynacore/cpu/qmm.h:125-126)
  * and DotQ8RowsNFn (dynacore/include/dynacore/cpu/cpu_kernels.h:53-54).
- * Any m: the weights are streamed once per pass of up to 4 activation rows. */
+ * Any m: the weights are streamed once per pass of up to 64 activation rows (by pair). */
 DQ_API int dq_gemv(const dq_weight* w, int fmt, const void* acts, int64_t m, int64_t n0, int64_t n1, float* y,
                    int64_t y_stride, const float* bias, void* stream);
 /* dq_gemm runs the prefill GEMMs on the matrix cores: Q4_K and Q6_K weights with
@@ -221,7 +221,7 @@ DQ_API int dq_gemm(const dq_weight* w, int fmt, const void* acts, int64_t m, int
 
 /* y = x . w^T (+ bias): quantize x with dq_act_format_for(w), then GEMV or GEMM by
  * m (Q4_K: GEMM above DQ_GEMV_MAX_ROWS, or above 48 rows for weights of <= 4096 rows;
- * Q8_0 / Q4_0: GEMM from 13 rows; Q6_K: GEMM
+ * Q8_0 / Q4_0: quantize + the MFMA GEMV from 3 or 5 rows by shape, GEMM from 13 rows; Q6_K: GEMM
  * above 64 rows, or above 16 for weights of >= 4096 rows or long K, except long rows on
  * weights of few rows, which run the 16-row skinny GEMV per 16 rows). Every route gives
  * the same bits. Replaces Device::matmul

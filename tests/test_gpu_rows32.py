@@ -1,0 +1,111 @@
+"""The MFMA GEMV of Q8_0 / Q4_0 weights x per-32 rows (dq_rows32.hip) and its route."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import dynalm_amd as dq
+from dqtest import activations, gguf_weights, weight_rows
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+TYPES32 = [O.Q8_0, O.Q4_0]
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+def check(t, rows, x, k, y, bias=None):
+    acts = O.quantize_act(O.ACT_PER32, x)
+    want = O.matmul(t, O.ACT_PER32, rows, acts, k).astype(np.float64)
+    mag = np.abs(x.astype(np.float64)) @ np.abs(O.expand_x86(t, rows, k).astype(np.float64)).T
+    b = 0.0 if bias is None else bias
+    # K / 32 terms, each and each partial sum rounded once, in two orders; codes are up to half
+    # a step above |x|
+    bound = (k / 32 + 16) * 2.0**-23 * 1.1 * (mag + np.abs(b) + np.abs(want))
+    assert np.all(np.abs(y - (want + b)) <= bound + 1e-30)
+
+
+# m, n, K: 16-, 32- and 64-row workgroups (tiles of 16 rows against 1.5 and 3 per CU), one
+# block to a partial last step of four, one to three passes with a short last one
+@pytest.mark.parametrize("t", TYPES32, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("m,n,k", [(3, 1, 32), (4, 17, 64), (5, 130, 96), (16, 63, 1312), (17, 200, 2048), (12, 4100, 160),
+                                   (8, 6200, 256), (5, 12300, 288), (11, 14336, 128), (48, 65, 8192), (33, 40, 8224)])
+def test_against_oracle(cuda, t, m, n, k):
+    import dqtorch as T
+
+    rows = gguf_weights(t, n, k, 6100 + t + m)
+    x = activations(m, k, 6200 + m)
+    bias = O.normal(6300 + m, n)
+    w = dq.Weight.upload(t, rows, k)
+    xs = np.zeros((m, k + 5), np.float32)
+    xs[:, :k] = x
+    xd = dev(xs)
+    y = torch.zeros((m, n + 3), device="cuda")
+    dq.matmul(w, xd, m, k + 5, y, n + 3, dev(bias), T.stream())
+    got = host(y)
+    assert not got[:, n:].any()
+    check(t, rows, x, k, got[:, :n], bias)
+    # the same bits from separately quantized rows (the GEMM's own from 13), and for any range
+    # of weight rows
+    acts = T.quantize(O.ACT_PER32, xd[:, :k].contiguous())
+    z = torch.zeros((m, n), device="cuda")
+    dq.gemv(w, dq.ACT_PER32, acts, m, 0, n, z, n, dev(bias), T.stream())
+    full = host(z).copy()
+    check(t, rows, x, k, full, bias)
+    if m < 13:
+        assert np.array_equal(full.view(np.uint32), got[:, :n].copy().view(np.uint32))
+    n0, n1 = n // 3, n - n // 4
+    z.zero_()
+    dq.gemv(w, dq.ACT_PER32, acts, m, n0, n1, z, n, dev(bias), T.stream())
+    part = host(z)
+    assert np.array_equal(part[:, n0:n1].copy().view(np.uint32), full[:, n0:n1].copy().view(np.uint32))
+    assert not part[:, :n0].any() and not part[:, n1:].any()
+
+
+@pytest.mark.parametrize("t", TYPES32, ids=lambda t: O.TYPE_NAMES[t])
+def test_saturated_codes(cuda, t):
+    """Edge weight blocks (extreme codes and scales) against rows of full-scale codes."""
+    import dqtorch as T
+
+    m, n, k = 9, 64, 1024
+    rows = weight_rows(t, n, k, 6400 + t, edge=True)
+    x = np.where(np.arange(m * k).reshape(m, k) % 3 == 0, -1.0, 1.0).astype(np.float32)
+    x[4] = 0.0
+    w = dq.Weight.upload(t, rows, k)
+    got = host(T.matmul(w, dev(x)))
+    want = O.matmul(t, O.ACT_PER32, rows, O.quantize_act(O.ACT_PER32, x), k).astype(np.float64)
+    mag = np.abs(x.astype(np.float64)) @ np.abs(O.expand_x86(t, rows, k).astype(np.float64)).T
+    fine = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fine)
+    assert np.all(np.abs(got - want)[fine] <= ((k / 32 + 16) * 2.0**-23 * 2 * mag + 1e-30)[fine])
+
+
+def test_first_call_under_capture(cuda):
+    """A stream whose workspace is not there yet and cannot be allocated (capture): the call
+    still runs, on the GEMV that needs none; three replays beside eager work."""
+    m, n, k = 8, 300, 512
+    rows = gguf_weights(O.Q4_0, n, k, 6500)
+    w = dq.Weight.upload(O.Q4_0, rows, k)
+    x = activations(m, k, 6501)
+    xd, y, e = dev(x), torch.zeros((m, n), device="cuda"), torch.zeros((m, n), device="cuda")
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        dq.matmul(w, xd, m, k, y, n, None, torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        check(O.Q4_0, rows, x, k, host(y))
+        dq.matmul(w, xd, m, k, e, n, None, torch.cuda.current_stream().cuda_stream)
+        check(O.Q4_0, rows, x, k, host(e))
