@@ -1044,7 +1044,7 @@ int dq_matmul_many(const dq_matmul_job* jobs, int64_t n_jobs, void* stream) {
   hipStream_t s = as_stream(stream);
   // the grouped jobs: decode-sized K-quant matmuls (the skinny MFMA GEMV, which
   // quantizes each job's fp32 rows itself); one launch per k for up to 8 jobs
-  std::vector<dq::GemvJob> grouped;
+  std::vector<dq::GemvJob> grouped, ones;
   std::vector<int64_t> others;
   for (int64_t i = 0; i < n_jobs; ++i) {
     const dq_matmul_job& j = jobs[i];
@@ -1052,9 +1052,33 @@ int dq_matmul_many(const dq_matmul_job* jobs, int64_t n_jobs, void* stream) {
     if (skinny_ok(j.w, j.x, j.m, j.x_stride)) {
       grouped.push_back(dq::GemvJob{&j.w->dev, nullptr, 0, j.x, j.m > 1 ? j.x_stride : j.w->dev.k, j.m, j.y,
                                     j.y_stride, j.bias});
+    } else if (j.m == 1 && dq::gemv_many_ok(j.w->dev)) {
+      ones.push_back(dq::GemvJob{&j.w->dev, nullptr, 0, j.x, j.w->dev.k, 1, j.y, j.y_stride, j.bias});
     } else {
       others.push_back(i);
     }
+  }
+  // one-row K-quant jobs of one k: one launch for up to kGemvManyMax (a single one as
+  // dq_matmul runs it)
+  while (!ones.empty()) {
+    dq::GemvJob batch[dq::kGemvManyMax];
+    int n = 0;
+    const int64_t nblk = ones[0].w->nblk;
+    std::vector<dq::GemvJob> rest;
+    for (const dq::GemvJob& j : ones) {
+      if (n < dq::kGemvManyMax && j.w->nblk == nblk) {
+        batch[n++] = j;
+      } else {
+        rest.push_back(j);
+      }
+    }
+    if (n > 1) {
+      DQ_HIP(dq::launch_gemv_many(batch, n, s), "grouped gemv launch");
+    } else {
+      DQ_HIP(dq::launch_gemv_fused(*batch[0].w, batch[0].x, batch[0].xs, 1, batch[0].y, batch[0].ys, batch[0].bias, s),
+             "gemv launch");
+    }
+    ones.swap(rest);
   }
   if (int rc = run_skinny(grouped, jobs[0].w->dev.device, s, dq::Region{}); rc != DQ_OK) return rc;
   for (int64_t i : others) {

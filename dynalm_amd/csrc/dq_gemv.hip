@@ -892,17 +892,15 @@ DQ_DEV void quantize_slice(const float* __restrict__ x, int64_t xs, int nblk, in
 // shape (the up projection); waves W/2.. run it over the same row group with their
 // own LDS regions, and y = act(x . gate) * (x . up) (dynacore's Device::matmul_gated,
 // dynacore/include/dynacore/device/device.h:188-199).
+// wg: the workgroup's index in its matmul (k_gemv: the grid's).
 template <int WT, int AF, int M, int W, int U, bool kFuse, int kEarly, bool kGated = false, bool kSplit = false>
-__global__ __launch_bounds__(W * 64) void k_gemv(const uint8_t* __restrict__ p0, const uint8_t* __restrict__ p1,
-                                                 const uint8_t* __restrict__ p2, const uint8_t* __restrict__ p3,
-                                                 int nblk, int64_t g0, int64_t n0, int64_t n1,
-                                                 const uint8_t* __restrict__ acts, int64_t arb,
-                                                 const float* __restrict__ x, int64_t xs,
-                                                 float* __restrict__ y, int64_t ys, const float* __restrict__ bias,
-                                                 int32_t* __restrict__ dbg, int64_t dbg_n,
-                                                 const uint8_t* __restrict__ q0, const uint8_t* __restrict__ q1,
-                                                 const uint8_t* __restrict__ q2, const uint8_t* __restrict__ q3,
-                                                 int act, int splits, float* __restrict__ part) {
+DQ_DEV void gemv_body(unsigned wg, const uint8_t* __restrict__ p0, const uint8_t* __restrict__ p1,
+                      const uint8_t* __restrict__ p2, const uint8_t* __restrict__ p3, int nblk, int64_t g0, int64_t n0,
+                      int64_t n1, const uint8_t* __restrict__ acts, int64_t arb, const float* __restrict__ x, int64_t xs,
+                      float* __restrict__ y, int64_t ys, const float* __restrict__ bias, int32_t* __restrict__ dbg,
+                      int64_t dbg_n, const uint8_t* __restrict__ q0, const uint8_t* __restrict__ q1,
+                      const uint8_t* __restrict__ q2, const uint8_t* __restrict__ q3, int act, int splits,
+                      float* __restrict__ part) {
   extern __shared__ __align__(16) uint8_t smem[];
   constexpr bool kSb = AF == kActQ8_K || AF == kActSX;
   static_assert(!kGated || (kSb && M == 1 && kFuse), "the gated GEMV takes one fp32 row and K-quant weights");
@@ -916,8 +914,8 @@ __global__ __launch_bounds__(W * 64) void k_gemv(const uint8_t* __restrict__ p0,
   const int half = kGated && wave >= WH ? 1 : 0;
   const int wl = wave - half * WH;
   // split-K (splits > 1): workgroup L takes K-range L % splits of row group L / splits
-  const int sk = kSplit ? (int)(blockIdx.x % (unsigned)splits) : 0;
-  const int64_t G = g0 + (kSplit ? (int64_t)(blockIdx.x / (unsigned)splits) : (int64_t)blockIdx.x);
+  const int sk = kSplit ? (int)(wg % (unsigned)splits) : 0;
+  const int64_t G = g0 + (kSplit ? (int64_t)(wg / (unsigned)splits) : (int64_t)wg);
   const size_t region = kSb ? ((size_t)M * nblk * 65 * 4 + 15) / 16 * 16 : (size_t)W * M * 64 * 4;
   Out<M> o;
   o.rec = reinterpret_cast<float*>(smem + half * region);
@@ -1086,6 +1084,58 @@ __global__ __launch_bounds__(W * 64) void k_gemv(const uint8_t* __restrict__ p0,
     } else {
       if (n >= n0 && n < n1) y[mm * ys + n] = bias ? v + bias[n] : v;
     }
+  }
+}
+
+template <int WT, int AF, int M, int W, int U, bool kFuse, int kEarly, bool kGated = false, bool kSplit = false>
+__global__ __launch_bounds__(W * 64) void k_gemv(const uint8_t* __restrict__ p0, const uint8_t* __restrict__ p1,
+                                                 const uint8_t* __restrict__ p2, const uint8_t* __restrict__ p3,
+                                                 int nblk, int64_t g0, int64_t n0, int64_t n1,
+                                                 const uint8_t* __restrict__ acts, int64_t arb,
+                                                 const float* __restrict__ x, int64_t xs,
+                                                 float* __restrict__ y, int64_t ys, const float* __restrict__ bias,
+                                                 int32_t* __restrict__ dbg, int64_t dbg_n,
+                                                 const uint8_t* __restrict__ q0, const uint8_t* __restrict__ q1,
+                                                 const uint8_t* __restrict__ q2, const uint8_t* __restrict__ q3,
+                                                 int act, int splits, float* __restrict__ part) {
+  gemv_body<WT, AF, M, W, U, kFuse, kEarly, kGated, kSplit>(blockIdx.x, p0, p1, p2, p3, nblk, g0, n0, n1, acts, arb, x,
+                                                            xs, y, ys, bias, dbg, dbg_n, q0, q1, q2, q3, act, splits,
+                                                            part);
+}
+
+// ---- one-row K-quant matmuls of one K in one launch (q, k and v of a decode step, the
+// experts of one token): the grid is the concatenation of the jobs' row groups, each
+// workgroup k_gemv's fused one-row body on its job, so every output has k_gemv's bits.
+// Such matmuls are launch-bound one by one: q / k / v at K = 1536 (1536, 256 and 256 rows)
+// took 11.9 us in three launches, 5.0 in one (graph replay); K = 4096 (4096, 1024, 1024) 13.8
+// against 5.6, (11008, 2753, 2753) 16.8 against 11.5; Q6_K K = 14336 (14336, 4096, 4096) 74 against
+// 56.
+struct OneRowJob {
+  const uint8_t* p[4];
+  const float* x;
+  float* y;
+  const float* bias;
+  int64_t n;
+  int dtype, wg0;  // wg0: the job's first workgroup
+};
+struct OneRowGroup {
+  OneRowJob job[kGemvManyMax];
+  int count, nblk;
+};
+template <int kEarly>
+__global__ __launch_bounds__(1024) void k_gemv_many(const OneRowGroup g) {
+  const int wg = (int)blockIdx.x;
+  int j = 0;
+  while (j + 1 < g.count && wg >= g.job[j + 1].wg0) ++j;
+  const OneRowJob& J = g.job[j];
+  if (J.dtype == kQ6_K) {
+    gemv_body<kQ6_K, kActQ8_K, 1, 16, 1, true, kEarly>(wg - J.wg0, J.p[0], J.p[1], J.p[2], J.p[3], g.nblk, 0, 0, J.n,
+                                                       nullptr, 0, J.x, 0, J.y, 0, J.bias, nullptr, 0, nullptr, nullptr,
+                                                       nullptr, nullptr, 0, 1, nullptr);
+  } else {
+    gemv_body<kQ4_K, kActQ8_K, 1, 16, 1, true, kEarly>(wg - J.wg0, J.p[0], J.p[1], J.p[2], J.p[3], g.nblk, 0, 0, J.n,
+                                                       nullptr, 0, J.x, 0, J.y, 0, J.bias, nullptr, 0, nullptr, nullptr,
+                                                       nullptr, nullptr, 0, 1, nullptr);
   }
 }
 
@@ -1492,6 +1542,48 @@ static hipError_t gemv_rows(const WeightDev& w, int af, const uint8_t* acts, int
     r0 += rows;
   }
   return hipSuccess;
+}
+
+template <int kEarly>
+static hipError_t many_launch(const OneRowGroup& g, int64_t wgs, size_t lds, hipStream_t s) {
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemv_many<kEarly>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemvMaxLds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_gemv_many<kEarly>), dim3((unsigned)wgs), dim3(1024), lds, s, g);
+  return hipGetLastError();
+}
+
+bool gemv_many_ok(const WeightDev& w) {
+  return (w.dtype == kQ4_K || w.dtype == kQ6_K) && w.nblk <= 64 &&
+         gemv_lds_bytes(w.dtype, kActQ8_K, 1, 16, w.nblk, true) <= kGemvMaxLds;
+}
+
+hipError_t launch_gemv_many(const GemvJob* jobs, int count, hipStream_t s) {
+  if (count < 1 || count > kGemvManyMax) return hipErrorInvalidValue;
+  OneRowGroup g{};
+  g.count = count;
+  g.nblk = (int)jobs[0].w->nblk;
+  int64_t wgs = 0;
+  size_t lds = 0;
+  for (int i = 0; i < count; ++i) {
+    const WeightDev& w = *jobs[i].w;
+    if (!gemv_many_ok(w) || w.nblk != g.nblk || jobs[i].m != 1 || jobs[i].x == nullptr) return hipErrorInvalidValue;
+    OneRowJob& j = g.job[i];
+    for (int p = 0; p < 4; ++p) j.p[p] = w.plane[p];
+    j.x = jobs[i].x;
+    j.y = jobs[i].y;
+    j.bias = jobs[i].bias;
+    j.n = w.n;
+    j.dtype = w.dtype;
+    j.wg0 = (int)wgs;
+    wgs += (w.n + kRowGroup - 1) / kRowGroup;
+    const size_t b = gemv_lds_bytes(w.dtype, kActQ8_K, 1, 16, w.nblk, true);
+    lds = b > lds ? b : lds;
+  }
+  if (wgs >= (1ll << 31)) return hipErrorInvalidValue;
+  if (g.nblk <= 16) return many_launch<1>(g, wgs, lds, s);
+  if (g.nblk <= 32) return many_launch<2>(g, wgs, lds, s);
+  return many_launch<4>(g, wgs, lds, s);
 }
 
 // The gated M = 1 GEMV: one workgroup per 64-row group holds both weights' rows,

@@ -218,6 +218,11 @@ struct GemvJob {
 // fused or none), Q4_K / Q6_K, 2 <= m <= 64 (fused: m <= 16), in launches of up to
 // 8 jobs; hipErrorInvalidValue for any other job.
 hipError_t launch_gemv_mma_many(const GemvJob* jobs, int count, hipStream_t s, const Workspace* ws = nullptr);
+// Up to kGemvManyMax one-row matmuls (m == 1, fp32 rows in GemvJob::x, K-quants of one K for
+// which gemv_many_ok) in one launch, each output with the one-row GEMV's bits.
+constexpr int kGemvManyMax = 8;
+bool gemv_many_ok(const WeightDev& w);
+hipError_t launch_gemv_many(const GemvJob* jobs, int count, hipStream_t s);
 // Work of one grouped launch of these jobs (<= 8, one nblk) in wave-sized units
 // (workgroups x super-blocks): each unit of a launch on fp32 rows quantizes 16
 // activation rows of one super-block again, so the caller quantizes once instead
