@@ -572,13 +572,16 @@ int matmul_act_impl(const dq_weight* w, int fmt, const float* x, int64_t m, int6
            "gemm launch");
     return DQ_OK;
   }
-  if (fmt == DQ_ACT_PER32 && (w->dev.dtype == DQ_Q4_K || w->dev.dtype == DQ_Q6_K) && m <= 8 &&
+  if (((fmt == DQ_ACT_PER32 && (w->dev.dtype == DQ_Q4_K || w->dev.dtype == DQ_Q6_K) && m <= 8) ||
+       (fmt == DQ_ACT_Q16 && gemv_fuses_q16(w->dev, m))) &&
       !use_gemm(w->dev, fmt, m)) {
-    // K-quants x per-32 decode (qmm's int8 gemv): one pass, each wave quantizing its
-    // slice with the standalone quantizer's arithmetic (the codes dq_act_quantize writes)
+    // K-quants x per-32 or int16 decode (qmm's gemv): one pass, each wave quantizing its
+    // slice with the standalone quantizer's arithmetic (the codes dq_act_quantize writes).
+    // int16, one row, against a quantize launch before it: Q6_K K = 14336, N = 4096 16.6 us (17.4),
+    // K = 8960, N = 1536 11.9 (13.2); Q4_K K = 4096, N = 14336 9.0 (10.6), 4 rows N = 4096 15.0 (16.6)
     const Workspace ws = split_ws(r, 0);
     DQ_HIP(launch_gemv_fused(w->dev, x, m > 1 ? x_stride : w->dev.k, m, y, y_stride, bias, s, r.base ? &ws : nullptr,
-                             kActPer32),
+                             fmt),
            "gemv launch");
     return DQ_OK;
   }

@@ -868,6 +868,24 @@ DQ_DEV void quantize_slice(const float* __restrict__ x, int64_t xs, int nblk, in
       for (int mm = 0; mm < M; ++mm) {
         float d;
         int sum;
+        if constexpr (AF == kActQ16) {
+          // the codes' bytes and the stored codes' sums of values 0..15 and 16..31, as stage_acts
+          const v2u c = q16_quant(v[mm], d, sum);
+          int a16 = sdot2w(c.y, sdot2w(c.x, 0));
+          a16 += dpp<kQuadXor1>(a16);
+          a16 += dpp<kQuadXor2>(a16);
+          if (blk < e1) {
+            uint8_t* o = st + (mm * nblk * bpu + blk) * kStage16;
+            *reinterpret_cast<u32*>(o + 16 + 4 * (r & 7)) = __builtin_amdgcn_perm(c.y, c.x, 0x07050301u);
+            *reinterpret_cast<u32*>(o + 48 + 4 * (r & 7)) = __builtin_amdgcn_perm(c.y, c.x, 0x06040200u);
+            if ((r & 3) == 0) *reinterpret_cast<int32_t*>(o + 8 + (r & 4)) = a16;
+            if ((r & 7) == 0) {
+              *reinterpret_cast<float*>(o) = d;
+              *reinterpret_cast<int32_t*>(o + 4) = sum;
+            }
+          }
+          continue;
+        }
         const u32 packed = per32_quant(v[mm], d, sum);
         if (blk < e1) {
           uint8_t* o = st + (mm * nblk * bpu + blk) * kStage32;
@@ -904,8 +922,9 @@ DQ_DEV void gemv_body(unsigned wg, const uint8_t* __restrict__ p0, const uint8_t
   extern __shared__ __align__(16) uint8_t smem[];
   constexpr bool kSb = AF == kActQ8_K || AF == kActSX;
   static_assert(!kGated || (kSb && M == 1 && kFuse), "the gated GEMV takes one fp32 row and K-quant weights");
-  static_assert((AF != kActSX && AF != kActQ16 && AF != kActF32) || (!kFuse && kEarly == 0),
-                "sub-scaled, int16 and fp32 activations arrive ready and are staged by loops");
+  static_assert((AF != kActSX && AF != kActF32) || !kFuse, "sub-scaled and fp32 activations arrive ready");
+  static_assert((AF != kActSX && AF != kActQ16 && AF != kActF32) || kEarly == 0,
+                "sub-scaled, int16 and fp32 activations are staged by loops");
   // LDS: Q8_K t-terms [M][nblk][64] + da [M][nblk]  |  per-32 slice sums [W][M][64];
   // then the staged activation rows [M][nblk (blocks of 32 for per-32)][stage bytes].
   // kGated: one t-term region and one stage region per weight.
@@ -1469,9 +1488,15 @@ static hipError_t gemv_pass(const WeightDev& w, int af, const uint8_t* acts, int
   if (x != nullptr) {
     switch (w.dtype) {
       case kQ4_K:
+        if constexpr (M <= 4) {
+          if (af == kActQ16) return gemv_waves<kQ4_K, kActQ16, M, true>(w, nullptr, 0, x, xs, n0, n1, y, ys, bias, dbg, ws, s);
+        }
         if (af == kActPer32) return gemv_waves<kQ4_K, kActPer32, M, true>(w, nullptr, 0, x, xs, n0, n1, y, ys, bias, dbg, ws, s);
         return gemv_waves<kQ4_K, kActQ8_K, M, true>(w, nullptr, 0, x, xs, n0, n1, y, ys, bias, dbg, ws, s);
       case kQ6_K:
+        if constexpr (M <= 2) {
+          if (af == kActQ16) return gemv_waves<kQ6_K, kActQ16, M, true>(w, nullptr, 0, x, xs, n0, n1, y, ys, bias, dbg, ws, s);
+        }
         if (af == kActPer32) return gemv_waves<kQ6_K, kActPer32, M, true>(w, nullptr, 0, x, xs, n0, n1, y, ys, bias, dbg, ws, s);
         return gemv_waves<kQ6_K, kActQ8_K, M, true>(w, nullptr, 0, x, xs, n0, n1, y, ys, bias, dbg, ws, s);
       case kQ8_0: return gemv_waves<kQ8_0, kActPer32, M, true>(w, nullptr, 0, x, xs, n0, n1, y, ys, bias, dbg, ws, s);
@@ -1636,9 +1661,17 @@ hipError_t launch_gemv(const WeightDev& w, int af, const uint8_t* acts, int64_t 
   return gemv_rows(w, af, acts, arb, nullptr, 0, m, n0, n1, y, ys, bias, dbg, ws, s);
 }
 
+// (the rows from which dq_matmul_act's int16 GEMMs take over are 5 and 3)
+bool gemv_fuses_q16(const WeightDev& w, int64_t m) {
+  if (m < 1 || m > (w.dtype == kQ4_K ? 4 : w.dtype == kQ6_K ? 2 : 0)) return false;
+  return gemv_lds_bytes(w.dtype, kActQ16, (int)m, 16, w.nblk, false) <= kGemvMaxLds;
+}
+
 hipError_t launch_gemv_fused(const WeightDev& w, const float* x, int64_t xs, int64_t m, float* y, int64_t ys,
                              const float* bias, hipStream_t s, const Workspace* ws, int af) {
-  if (af >= 0 && !(af == kActPer32 && (w.dtype == kQ4_K || w.dtype == kQ6_K))) return hipErrorInvalidValue;
+  if (af >= 0 && !(af == kActPer32 && (w.dtype == kQ4_K || w.dtype == kQ6_K)) && !(af == kActQ16 && gemv_fuses_q16(w, m))) {
+    return hipErrorInvalidValue;
+  }
   return gemv_rows(w, af, nullptr, 0, x, xs, m, 0, w.n, y, ys, bias, nullptr, ws, s);
 }
 

@@ -72,10 +72,12 @@ hipError_t launch_gemv(const WeightDev& w, int af, const uint8_t* acts, int64_t 
                        const Workspace* ws = nullptr);
 // Decode matmul with the activation quantization fused into the GEMV (fp32 rows x,
 // row stride xs floats): af < 0, the weight's activation format (dq_act_format_for);
-// af = kActPer32 for Q4_K / Q6_K, per-32 rows (qmm's int8 contract), each wave
-// quantizing its slice with the standalone per-32 quantizer's device function.
+// af = kActPer32 or kActQ16 for Q4_K / Q6_K, per-32 or int16 rows (qmm's contracts), each
+// wave quantizing its slice with the standalone quantizer's device function.
 hipError_t launch_gemv_fused(const WeightDev& w, const float* x, int64_t xs, int64_t m, float* y, int64_t ys,
                              const float* bias, hipStream_t s, const Workspace* ws = nullptr, int af = -1);
+// Whether launch_gemv_fused takes m rows of w with af = kActQ16 (one pass).
+bool gemv_fuses_q16(const WeightDev& w, int64_t m);
 // K-ranges per row of the GEMV on this weight under activation format af (1: no
 // split-K), and the bytes of row sums a pass of up to m_pass rows then needs (0 when
 // it does not split). Both depend on the weight and the device only.
