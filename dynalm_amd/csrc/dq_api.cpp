@@ -175,14 +175,10 @@ int with_stream_ws(int device, void* stream, size_t need, F&& fn) {
   return fn(static_cast<uint8_t*>(e->p));
 }
 
-// Whether with_stream_ws can serve `need` bytes now: the stream's workspace holds them or may
-// grow, which a stream under capture may not.
-bool stream_ws_ready(int device, void* stream, size_t need) {
-  {
-    std::lock_guard<std::mutex> lock(g_sws_mu);
-    for (const StreamWs& x : g_sws)
-      if (x.device == device && x.stream == stream && x.bytes >= need) return true;
-  }
+// Whether the stream is not capturing: a captured launch keeps its buffers' addresses, and a
+// later call may grow (free) the stream's workspace, so a route that can do without one does
+// under capture.
+bool not_capturing(void* stream) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(as_stream(stream), &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
   (void)hipGetLastError();  // not this call's error: the launches after it report their own
@@ -512,8 +508,8 @@ int matmul_impl(const dq_weight* w, const float* x, int64_t m, int64_t x_stride,
   }
   if (rows32_pays(w->dev, fmt, m) && !use_gemm(w->dev, fmt, m)) {
     // Q8_0 / Q4_0 decode batches: quantize once, then the MFMA GEMV. The rows go to the
-    // region or this stream's workspace; where there is no room and none can be allocated (a
-    // stream under capture), the routes below
+    // region or this stream's workspace; without room, or under capture without a region, the
+    // routes below
     const int64_t need = m * arb;
     auto run = [&](uint8_t* p) -> int {
       DQ_HIP(launch_quantize(fmt, x, m, w->dev.k, m > 1 ? x_stride : w->dev.k, p, arb, s), "quantize launch");
@@ -522,7 +518,7 @@ int matmul_impl(const dq_weight* w, const float* x, int64_t m, int64_t x_stride,
     };
     if (r.base != nullptr) {
       if ((size_t)need <= r.bytes) return run(r.base);
-    } else if (need < ((int64_t)1 << 32) && m <= 65535 && stream_ws_ready(w->dev.device, stream, (size_t)need)) {
+    } else if (need < ((int64_t)1 << 32) && m <= 65535 && not_capturing(stream)) {
       return with_stream_ws(w->dev.device, stream, (size_t)need, run);
     }
   }

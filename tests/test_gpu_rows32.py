@@ -109,3 +109,32 @@ def test_first_call_under_capture(cuda):
         check(O.Q4_0, rows, x, k, host(y))
         dq.matmul(w, xd, m, k, e, n, None, torch.cuda.current_stream().cuda_stream)
         check(O.Q4_0, rows, x, k, host(e))
+
+
+@pytest.mark.parametrize("t", TYPES32, ids=lambda t: O.TYPE_NAMES[t])
+def test_capture_outlives_the_stream_workspace(cuda, t):
+    """A call captured on a stream that has a workspace does not use it: the graph replays
+    right after a larger call on the stream has replaced the workspace."""
+    import dqtorch as T
+
+    m, n, k, kb = 8, 300, 512, 14336
+    rows, big = gguf_weights(t, n, k, 6600 + t), gguf_weights(O.Q4_K, 64, kb, 6610)
+    w, wb = dq.Weight.upload(t, rows, k), dq.Weight.upload(O.Q4_K, big, kb)
+    x = activations(m, k, 6601)
+    xd, y, e = dev(x), torch.zeros((m, n), device="cuda"), torch.zeros((m, n), device="cuda")
+    # dq_gemm's activation layouts: 2 B a value and more in the stream's workspace, 7 MB and up
+    acts = [T.quantize(O.ACT_PER32, torch.ones((b, kb), device="cuda")) for b in (256, 512, 1024)]
+    yb = torch.zeros((1024, 64), device="cuda")
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    dq.matmul(w, xd, m, k, e, n, None, s.cuda_stream)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        dq.matmul(w, xd, m, k, y, n, None, s.cuda_stream)
+    for a in acts:
+        dq.gemm(wb, dq.ACT_PER32, a, a.shape[0], 0, 64, yb, 64, None, s.cuda_stream)
+        torch.cuda.synchronize()
+        y.zero_()
+        g.replay()
+        check(t, rows, x, k, host(y))
