@@ -12,8 +12,8 @@
 // whole load (Q8_0: two) of its row, with no exchange between lanes, and a lane's activation
 // operand is a whole block of its activation row. Block g's dot is the MFMA with the
 // activation operand zeroed outside group g (eight `and`s a block, shared by the step's TC
-// weight tiles); t = dw da of all 16 x 16 outputs is one v_mfma_f32_16x16x4_f32 on the scales
-// masked alike (one product per output, rounded once); Q4_0's -8 sum(a) is the same MFMA
+// weight tiles); t = dw da of the four blocks' 16 x 16 outputs is one v_mfma_f32_16x16x1_4b_f32 on
+// the scales, group g's for block g (one product per output, rounded once); Q4_0's -8 sum(a) is the same MFMA
 // against a constant -8, once per block, as the accumulator the tiles start from. That leaves 8
 // VALU per block and tile (convert, fma) and Q4_0's 12 to split nibbles.
 //
