@@ -104,8 +104,8 @@ __global__ __launch_bounds__(64 * W) void k_rows32(const uint8_t* __restrict__ p
     gb[i] = (u32)((n >> 6) * nblk);
     r[i] = (u32)(n & 63);
   }
-  // rows past m repeat the last one (their outputs are not stored); blocks past K too (their
-  // weights are zero)
+  // rows past m repeat the last one (their outputs are not stored); blocks past K repeat the last
+  // one's codes, with weights and scales of zero (an infinite scale times a zero weight is NaN)
   const uint8_t* row = acts + (int64_t)(c < m ? c : m - 1) * stride;
   auto ablk = [&](int q) { return 4 * q + g < nblk ? 4 * q + g : nblk - 1; };
 
@@ -118,6 +118,7 @@ __global__ __launch_bounds__(64 * W) void k_rows32(const uint8_t* __restrict__ p
   ActRaw a[2];
   auto load = [&](int q, int set) {
     a[set].load(row, ablk(q));
+    if (4 * q + g >= nblk) a[set].d = 0.0f;
 #pragma unroll
     for (int i = 0; i < TC; ++i) w[set][i].load(rq, rd, gb[i], r[i], 4 * q + g, nblk);
   };

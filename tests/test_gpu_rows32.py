@@ -90,6 +90,29 @@ def test_saturated_codes(cuda, t):
     assert np.all(np.abs(got - want)[fine] <= ((k / 32 + 16) * 2.0**-23 * 2 * mag + 1e-30)[fine])
 
 
+@pytest.mark.parametrize("t", TYPES32, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("k", [96, 128, 160, 224])
+def test_infinite_last_block(cuda, t, k):
+    """An infinity or a NaN in a row's last block, which the lanes of a short last step repeat:
+    each output is the infinity or NaN that the contract's order and the one-row call give."""
+    import dqtorch as T
+
+    m, n = 12, 64
+    rows = gguf_weights(t, n, k, 6700 + t)
+    x = activations(m, k, 6701)
+    x[1, k - 3], x[2, k - 5], x[3, k - 1], x[4, 0] = np.inf, -np.inf, np.nan, np.inf
+    w = dq.Weight.upload(t, rows, k)
+    want = O.matmul(t, O.ACT_PER32, rows, O.quantize_act(O.ACT_PER32, x), k)
+    one = np.concatenate([host(T.matmul(w, dev(x[r : r + 1]))).copy() for r in range(m)])
+    for rr in (3, 5, 8, m):
+        got = host(T.matmul(w, dev(x[:rr])))
+        for ref in (want[:rr], one[:rr]):
+            odd = ~np.isfinite(ref)
+            assert np.array_equal(~np.isfinite(got), odd)
+            assert np.array_equal(got[odd], ref[odd], equal_nan=True)
+    assert np.isinf(want).any()
+
+
 def test_first_call_under_capture(cuda):
     """A stream whose workspace is not there yet and cannot be allocated (capture): the call
     still runs, on the GEMV that needs none; three replays beside eager work."""
