@@ -1328,6 +1328,10 @@ int gemv_splits(const WeightDev& w, int af) {
   return splits;
 }
 
+int gemv_waves32(const WeightDev& w, int af) {
+  return gemv_splits(w, af) == 1 && w.n_pad / kRowGroup <= w.cus ? 16 : 8;
+}
+
 size_t gemv_split_bytes(const WeightDev& w, int af, int64_t m_pass) {
   const int splits = gemv_splits(w, af);
   return splits > 1 ? (size_t)(w.n_pad / kRowGroup) * splits * (size_t)m_pass * 64 * 4 : 0;
@@ -1474,7 +1478,7 @@ static hipError_t gemv_waves(const WeightDev& w, const uint8_t* acts, int64_t ar
     }
   }
   const Split none;
-  if (kWide && groups <= w.cus) {
+  if (kWide && gemv_waves32(w, AF) == 16) {
     return gemv_early<WT, AF, M, kFuse, kWide ? 16 : 8, false>(w, acts, arb, x, xs, n0, n1, y, ys, bias, dbg, none, s);
   }
   return gemv_early<WT, AF, M, kFuse, 8, false>(w, acts, arb, x, xs, n0, n1, y, ys, bias, dbg, none, s);

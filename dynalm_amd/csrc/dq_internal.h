@@ -82,6 +82,9 @@ bool gemv_fuses_q16(const WeightDev& w, int64_t m);
 // split-K), and the bytes of row sums a pass of up to m_pass rows then needs (0 when
 // it does not split). Both depend on the weight and the device only.
 int gemv_splits(const WeightDev& w, int af);
+// K slices of such a range, one per wave: 16 where a row has one range and all row groups fit on
+// the CUs at once, else 8 (K-quant passes of several rows: always 8).
+int gemv_waves32(const WeightDev& w, int af);
 size_t gemv_split_bytes(const WeightDev& w, int af, int64_t m_pass);
 hipError_t launch_units(const WeightDev& w, int af, const uint8_t* acts, int64_t arb, int64_t m, int32_t* units,
                         int64_t nu, hipStream_t s);

@@ -2,31 +2,36 @@
 // weights x per-32 activations for 2..16 activation rows per pass, on int8 MFMA.
 //
 // Arithmetic per output and 32-value block b (kernels_generic.cpp:210-239): P_b, the exact
-// integer dot of the codes (Q4_0: nibble - 8), t = dw_b da_b rounded to fp32, acc = fma(t,
-// (float)P_b, acc) over the blocks of a wave's slice in order, the slices added in order. The
-// slices depend on K only, so an output's bits depend neither on the row range nor on m.
+// integer dot of the codes (Q4_0: nibble - 8), t = dw_b da_b rounded to fp32, acc = acc + t
+// (float)P_b over the blocks of a K slice in order, the slices added in order. Slices and roundings
+// are the VALU GEMV's (gemv_splits ranges of gemv_waves32 slices), so an output has the same bits
+// from either kernel, whatever the row count, the row range or the route.
 //
 // MFMA mapping (v_mfma_i32_16x16x64_i8: lane l supplies row / column l % 16 and 16 K values of
 // lane group l / 16; result lane l holds column l % 16, rows 4 (l / 16) .. + 3). A step takes
-// four blocks, lane group g holding block 4 q + g: a lane's 16 bytes of weights are then one
-// whole load (Q8_0: two) of its row, with no exchange between lanes, and a lane's activation
-// operand is a whole block of its activation row. Block g's dot is the MFMA with the
-// activation operand zeroed outside group g (eight `and`s a block, shared by the step's TC
-// weight tiles); t = dw da of the four blocks' 16 x 16 outputs is one v_mfma_f32_16x16x1_4b_f32 on
-// the scales, group g's for block g (one product per output, rounded once); Q4_0's -8 sum(a) is the same MFMA
-// against a constant -8, once per block, as the accumulator the tiles start from. That leaves 8
-// VALU per block and tile (convert, fma) and Q4_0's 12 to split nibbles.
+// four blocks, one per lane group: a lane's 16 bytes of weights are then one whole load (Q8_0:
+// two) of its row, with no exchange between lanes, and a lane's activation operand is a whole
+// block of its activation row. Block g's dot is the MFMA with the activation operand zeroed
+// outside group g (eight `and`s a block, shared by the step's TC weight tiles); t = dw da of the
+// four blocks' 16 x 16 outputs is one v_mfma_f32_16x16x1_4b_f32 on the scales, group g's for block
+// g (one product per output, rounded once); Q4_0's -8 sum(a) is the same MFMA against a constant
+// -8, once per block, as the accumulator the tiles start from. That leaves 12 VALU per block and
+// tile (convert, multiply, add) and Q4_0's 12 a step to split nibbles.
 //
 // The activations come quantized (one launch for the call): quantizing a lane's own block in
 // here, 32 values at ~8 VALU each in every workgroup, took 19.6 us a call against 15.
 //
-// Work split: a workgroup owns 16 TC weight rows and all of K, its W waves contiguous slices;
-// TC = 4 (the weight load instructions read 1 KB runs, the activations are prepared once per
-// 64 weight rows) while those workgroups fill the CUs, else 2 or 1.
-// What bounds it: Q4_0 K = 4096, N = 14336 at 8 rows takes 13 us for 33 MB (2.5 TB/s; before,
-// the VALU GEMV's dots of every row: 17.6). A wave's step is 48 MFMAs (~770 clocks) and ~236 VALU
-// (~940), so a workgroup's two waves per SIMD compute for ~4 us of it; two or one row of loads
-// in flight and 8 or 16 waves measured alike.
+// Work split: a workgroup owns 16 TC weight rows and all of K; TC = 4 (the weight load
+// instructions read 1 KB runs, the activations are prepared once per 64 weight rows) while those
+// workgroups fill the CUs, else 2 or 1. A wave's slices are contiguous in K. Of two short slices
+// (16 of a whole row) each takes two lane groups, which leaves no lane group idle at a slice's end;
+// one after the other they took 4.1 us instead of 3.3 at K = 1024, N = 4096. The long rows of
+// few row groups (two ranges and more) go slice by slice: a load of four consecutive blocks
+// touches half the cache lines of four slices' (Q8_0 K = 14336, N = 5120 at 8 rows 30.3 us
+// against 34.2), on 16 waves where one workgroup fills a CU (N = 2048, Q4_0 14.6 against 16.6).
+// What bounds it: Q4_0 K = 4096, N = 14336 at 8 rows takes 10.8 us for 33 MB (3.1 TB/s; the
+// VALU GEMV, which pays its dots for every row, 15.3). A wave's two steps per slice pair are 48
+// MFMAs and ~300 VALU each; loads one or two steps ahead measured alike.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -67,9 +72,9 @@ template <int WT>
 struct WBlk {
   v4u q[WT == kQ8_0 ? 2 : 1];
   u32 d;
-  DQ_DEV void load(__amdgpu_buffer_rsrc_t rq, __amdgpu_buffer_rsrc_t rd, u32 gb, u32 r, int b, int nblk) {
+  DQ_DEV void load(__amdgpu_buffer_rsrc_t rq, __amdgpu_buffer_rsrc_t rd, u32 gb, u32 r, int b, int end) {
     const u32 blk = gb + (u32)b;
-    const bool in = b < nblk;
+    const bool in = b < end;
     if constexpr (WT == kQ8_0) {
       q[0] = ld16nt(rq, in ? (blk * 2 * 64 + r) * 16 : kNoLoad);
       q[1] = ld16nt(rq, in ? ((blk * 2 + 1) * 64 + r) * 16 : kNoLoad);
@@ -84,13 +89,15 @@ struct WBlk {
 
 }  // namespace
 
-// Workgroup i: weight rows [16 (t0 + i TC), + 16 TC); acts: m <= 16 rows (fp32 or ActBlockQ8)
-// `stride` bytes apart.
-template <int WT, int TC, int W>
-__global__ __launch_bounds__(64 * W) void k_rows32(const uint8_t* __restrict__ p0, const uint8_t* __restrict__ p1,
-                                                   int nblk, int64_t n_pad, int64_t t0, int64_t n0, int64_t n1,
-                                                   const uint8_t* __restrict__ acts, int64_t stride, int m,
-                                                   float* __restrict__ y, int64_t ys, const float* __restrict__ bias) {
+// Workgroup i: weight rows [16 (t0 + i TC), + 16 TC); acts: m <= 16 ActBlockQ8 rows `stride`
+// bytes apart; kSplits K-ranges of WR slices. A wave's slices, contiguous in K, go in kRounds
+// rounds of G at once: the lane groups take 4 / G blocks of each of the G a step, `steps` steps a round.
+template <int WT, int TC, int kWaves, int kSplits, int WR, int G>
+__global__ __launch_bounds__(64 * kWaves) void k_rows32(const uint8_t* __restrict__ p0, const uint8_t* __restrict__ p1,
+                                                        int nblk, int64_t n_pad, int64_t t0, int64_t n0, int64_t n1,
+                                                        const uint8_t* __restrict__ acts, int64_t stride, int m,
+                                                        float* __restrict__ y, int64_t ys,
+                                                        const float* __restrict__ bias, int steps) {
   extern __shared__ __align__(16) float red[];
   const int t = threadIdx.x, lane = t & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -104,26 +111,58 @@ __global__ __launch_bounds__(64 * W) void k_rows32(const uint8_t* __restrict__ p
     gb[i] = (u32)((n >> 6) * nblk);
     r[i] = (u32)(n & 63);
   }
-  // rows past m repeat the last one (their outputs are not stored); blocks past K repeat the last
-  // one's codes, with weights and scales of zero (an infinite scale times a zero weight is NaN)
-  const uint8_t* row = acts + (int64_t)(c < m ? c : m - 1) * stride;
-  auto ablk = [&](int q) { return 4 * q + g < nblk ? 4 * q + g : nblk - 1; };
+  const uint8_t* row = acts + (int64_t)(c < m ? c : m - 1) * stride;  // rows past m repeat the last one (not stored)
 
-  const int nq = (nblk + 3) / 4, q0 = wave * nq / W, q1 = (wave + 1) * nq / W;
-  v4f_t acc[TC];
-#pragma unroll
-  for (int i = 0; i < TC; ++i) acc[i] = v4f_t{};
-  // two steps' loads in flight, quad q in set (q - q0) % 2
-  WBlk<WT> w[2][TC];
-  ActRaw a[2];
-  auto load = [&](int q, int set) {
-    a[set].load(row, ablk(q));
-    if (4 * q + g >= nblk) a[set].d = 0.0f;
-#pragma unroll
-    for (int i = 0; i < TC; ++i) w[set][i].load(rq, rd, gb[i], r[i], 4 * q + g, nblk);
+  // the lane group's slice of a round, [b, end); its block of step q is b + kB q
+  constexpr int kB = 4 / G, kPer = kSplits * WR / kWaves, kRounds = kPer / G;
+  static_assert(kPer * kWaves == kSplits * WR && kPer % G == 0, "whole rounds");
+  auto first = [&](int i) {  // the first block of slice i
+    const int sk = i / WR, wl = i % WR, k0 = sk * nblk / kSplits, k1 = (sk + 1) * nblk / kSplits;
+    return k0 + wl * (k1 - k0) / WR;
   };
-  if (q0 < q1) load(q0, 0);
-  if (q0 + 1 < q1) load(q0 + 1, 1);
+  int b, end;
+  auto round = [&](int r) {
+    const int i = kPer * wave + G * r + g / kB;
+    b = first(i) + g % kB;
+    end = first(i + 1);
+  };
+  round(0);
+  v4f_t acc[G][TC];
+#pragma unroll
+  for (int i = 0; i < G * TC; ++i) acc[i / TC][i % TC] = v4f_t{};
+  // the next kD steps' loads in flight (one where two would spill registers), step q in set q %
+  // kD; blocks past the slice repeat some block's codes, with weights and scales of zero (an
+  // infinite scale times a zero weight is NaN)
+  constexpr int kD = TC == 4 ? 1 : 2;
+  WBlk<WT> w[kD][TC];
+  ActRaw a[kD];
+  int lq = 0, lr = 0;  // the step to load: step lq of round lr
+  const int total = kRounds * steps;
+  auto load = [&](int set) {
+    a[set].load(row, b < nblk ? b : nblk - 1);
+    if (b >= end) a[set].d = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TC; ++i) w[set][i].load(rq, rd, gb[i], r[i], b, end);
+    b += kB;
+    if (kRounds > 1 && ++lq == steps) {
+      lq = 0;
+      round(++lr);
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < kD; ++q) {
+    if (q < total) load(q);
+  }
+  // a round's sums: element (tile i, lane, e) of slice j at ((j TC + i) 64 + lane) 4 + e
+  auto put_slices = [&](int r) {
+#pragma unroll
+    for (int i = 0; i < G * TC; ++i) {
+      *reinterpret_cast<v4f_t*>(red + (((kPer * wave + G * r + i / TC) * TC + i % TC) * 64 + lane) * 4) =
+          acc[i / TC][i % TC];
+      acc[i / TC][i % TC] = v4f_t{};
+    }
+  };
+  int cq = 0, cr = 0;  // the step to compute
   auto step = [&](int q, int set) {
     const ActBlk x = a[set].block();
     v4u lo[TC], hi[TC];
@@ -134,7 +173,7 @@ __global__ __launch_bounds__(64 * W) void k_rows32(const uint8_t* __restrict__ p
       hi[i] = w[set][i].hi();
       dw[i] = h2f(w[set][i].d);
     }
-    if (q + 2 < q1) load(q + 2, set);
+    if (q + kD < total) load(set);
     // t = dw da of the four blocks' 16 x 16 outputs: [block][4 rows]
     v16f_t sc[TC];
 #pragma unroll
@@ -151,39 +190,50 @@ __global__ __launch_bounds__(64 * W) void k_rows32(const uint8_t* __restrict__ p
 #pragma unroll
       for (int i = 0; i < TC; ++i) {
         const v4i_t P = mfma(ah, hi[i], mfma(al, lo[i], c0));
+        v4f_t& s = acc[gg / kB][i];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][e] = fmaf(sc[i][4 * gg + e], (float)P[e], acc[i][e]);
+        for (int e = 0; e < 4; ++e) s[e] = s[e] + sc[i][4 * gg + e] * (float)P[e];
       }
+    }
+    if (kRounds > 1 && ++cq == steps) {
+      put_slices(cr++);
+      cq = 0;
     }
   };
 #pragma unroll 1
-  for (int q = q0; q < q1; q += 2) {
+  for (int q = 0; q < total; q += kD) {
     step(q, 0);
-    if (q + 1 < q1) step(q + 1, 1);
+    if (kD == 2 && q + 1 < total) step(q + 1, kD - 1);
   }
+  if (kRounds == 1) put_slices(0);
 
-  // the waves' sums in wave order: element (tile i, lane, e) of wave v at ((v TC + i) 64 + lane) 4 + e
-#pragma unroll
-  for (int i = 0; i < TC; ++i) *reinterpret_cast<v4f_t*>(red + ((wave * TC + i) * 64 + lane) * 4) = acc[i];
+  // each K-range's slices in order, then the ranges
   __syncthreads();
-  for (int e = t; e < TC * 256; e += 64 * W) {
+  for (int e = t; e < TC * 256; e += 64 * kWaves) {
     const int l = (e >> 2) & 63, mr = 4 * (l >> 4) + (e & 3);
     const int64_t n = 16 * (tile0 + (e >> 8)) + (l & 15);
-    float v = red[e];
+    float v = 0;
+    for (int sk = 0; sk < kSplits; ++sk) {
+      float u = 0;
 #pragma unroll
-    for (int k = 1; k < W; ++k) v += red[k * TC * 256 + e];
+      for (int k = 0; k < WR; ++k) u = u + red[(sk * WR + k) * TC * 256 + e];
+      v = v + u;
+    }
     if (mr < m && n >= n0 && n < n1) y[mr * ys + n] = bias ? v + bias[n] : v;
   }
 }
 
 namespace {
 
-template <int WT, int TC, int W>
+template <int WT, int TC, int kWaves, int kSplits, int WR, int G>
 hipError_t launch1(const WeightDev& w, const uint8_t* acts, int64_t stride, int64_t m, int64_t n0, int64_t n1, float* y,
                    int64_t ys, const float* bias, hipStream_t s) {
+  static_assert(kSplits * WR * TC <= 64, "64 KB of LDS");
   const int64_t t0 = n0 / 16, wgs = ((n1 + 15) / 16 - t0 + TC - 1) / TC;
-  hipLaunchKernelGGL((k_rows32<WT, TC, W>), dim3((unsigned)wgs), dim3(64 * W), W * TC * 1024, s, w.plane[0],
-                     w.plane[1], (int)w.nblk, w.n_pad, t0, n0, n1, acts, stride, (int)m, y, ys, bias);
+  const int64_t range = (w.nblk + kSplits - 1) / kSplits, slice = (range + WR - 1) / WR;
+  hipLaunchKernelGGL((k_rows32<WT, TC, kWaves, kSplits, WR, G>), dim3((unsigned)wgs), dim3(64 * kWaves),
+                     kSplits * WR * TC * 1024, s, w.plane[0], w.plane[1], (int)w.nblk, w.n_pad, t0, n0, n1, acts,
+                     stride, (int)m, y, ys, bias, (int)((slice * G + 3) / 4));
   return hipGetLastError();
 }
 
@@ -191,9 +241,22 @@ template <int WT>
 hipError_t launch_type(const WeightDev& w, const uint8_t* acts, int64_t stride, int64_t m, int64_t n0, int64_t n1,
                        float* y, int64_t ys, const float* bias, hipStream_t s) {
   const int64_t tiles = w.n_pad / 16, cus = w.cus > 0 ? w.cus : 256;
-  if (tiles >= 3 * cus) return launch1<WT, 4, 8>(w, acts, stride, m, n0, n1, y, ys, bias, s);
-  if (2 * tiles >= 3 * cus) return launch1<WT, 2, 8>(w, acts, stride, m, n0, n1, y, ys, bias, s);
-  return launch1<WT, 1, 8>(w, acts, stride, m, n0, n1, y, ys, bias, s);
+  const int tc = tiles >= 3 * cus ? 4 : 2 * tiles >= 3 * cus ? 2 : 1;
+#define DQ_ROWS32(...) launch1<WT, __VA_ARGS__>(w, acts, stride, m, n0, n1, y, ys, bias, s)
+  switch (gemv_splits(w, kActPer32)) {
+    case 1:
+      if (gemv_waves32(w, kActPer32) == 8) return DQ_ROWS32(4, 8, 1, 8, 1);
+      return tc == 4 ? DQ_ROWS32(4, 8, 1, 16, 2) : tc == 2 ? DQ_ROWS32(2, 8, 1, 16, 2) : DQ_ROWS32(1, 8, 1, 16, 2);
+    case 2: return tc == 1 ? DQ_ROWS32(1, 8, 2, 8, 1) : DQ_ROWS32(2, 8, 2, 8, 1);
+    case 3: return DQ_ROWS32(1, 8, 3, 8, 1);
+    case 4: return DQ_ROWS32(1, 16, 4, 8, 1);
+    case 5: return DQ_ROWS32(1, 10, 5, 8, 1);
+    case 6: return DQ_ROWS32(1, 16, 6, 8, 1);
+    case 7: return DQ_ROWS32(1, 14, 7, 8, 1);
+    case 8: return DQ_ROWS32(1, 16, 8, 8, 1);
+    default: return hipErrorInvalidValue;
+  }
+#undef DQ_ROWS32
 }
 
 }  // namespace

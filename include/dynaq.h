@@ -224,8 +224,9 @@ DQ_API int dq_gemm(const dq_weight* w, int fmt, const void* acts, int64_t m, int
  * Q8_0 / Q4_0: quantize + the MFMA GEMV from 3 or 5 rows by shape, GEMM from 13 rows; Q6_K: GEMM
  * above 64 rows, or above 16 for weights of >= 4096 rows or long K, except long rows on
  * weights of few rows, which run the 16-row skinny GEMV per 16 rows). Every K-quant
- * route gives the same bits; the Q8_0 / Q4_0 routes add the blocks in orders of their own (under
- * stream capture 3..12 rows run the GEMV that needs no memory). Replaces Device::matmul
+ * route gives the same bits; so do the Q8_0 / Q4_0 GEMVs (up to 12 rows, whichever rows are beside
+ * a row; under stream capture they take the one that needs no memory), while their GEMM adds the
+ * blocks in another order. Replaces Device::matmul
  * (dynacore/include/dynacore/device/device.h:161; CpuDevice::matmul,
  * dynacore/cpu/cpu_device.cpp:869-1177). Uses a per-device scratch buffer. */
 DQ_API int dq_matmul(const dq_weight* w, const float* x, int64_t m, int64_t x_stride, float* y, int64_t y_stride,

@@ -113,6 +113,34 @@ def test_infinite_last_block(cuda, t, k):
     assert np.isinf(want).any()
 
 
+# N, K: every split of K -- 16 slices in 16-, 32- and 64-row workgroups, 8 slices (more row groups
+# than CUs), two to eight ranges of 8 -- with slices of no, a few and uneven blocks
+@pytest.mark.parametrize("t", TYPES32, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("n,k", [(70, 32), (300, 1504), (6200, 416), (14336, 96), (16500, 160), (6000, 8192), (7000, 8224),
+                                 (5000, 8192), (4096, 8288), (3100, 8192), (2600, 8224), (2304, 8192), (130, 14336)])
+def test_the_one_row_bits(cuda, t, n, k):
+    """A row's outputs are the one-row call's bit for bit whatever the rows beside it, from fp32 rows
+    and from quantized ones, and for rows whose scales and products fall below the normal range."""
+    import dqtorch as T
+
+    rows = gguf_weights(t, min(n, 128), k, 6800 + t)
+    rows = np.tile(rows, (-(-n // rows.shape[0]), 1))[:n].copy()
+    w = dq.Weight.upload(t, rows, k)
+    x = activations(16, k, 6801)
+    x[2] *= np.float32(1e-36)
+    x[5] *= np.float32(1e-39)
+    x[7] *= np.float32(1e34)
+    xd = dev(x)
+    acts = T.quantize(O.ACT_PER32, xd)
+    one = np.concatenate([host(T.matmul(w, xd[r : r + 1].contiguous())).copy() for r in range(16)])
+    for m in (3, 4, 5, 8, 12, 16):
+        z = torch.zeros((m, n), device="cuda")
+        dq.gemv(w, dq.ACT_PER32, acts, m, 0, n, z, n, None, T.stream())
+        assert np.array_equal(host(z).view(np.uint32), one[:m].view(np.uint32))
+        if m < 13:
+            assert np.array_equal(host(T.matmul(w, xd[:m].contiguous())).view(np.uint32), one[:m].view(np.uint32))
+
+
 def test_first_call_under_capture(cuda):
     """A stream whose workspace is not there yet and cannot be allocated (capture): the call
     still runs, on the GEMV that needs none; three replays beside eager work."""
