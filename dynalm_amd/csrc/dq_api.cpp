@@ -506,7 +506,7 @@ int matmul_impl(const dq_weight* w, const float* x, int64_t m, int64_t x_stride,
     if (int rc = dq_act_quantize(fmt, x, m, w->dev.k, x_stride, acts, stream); rc != DQ_OK) return rc;
     return dq_gemv(w, fmt, acts, m, 0, w->dev.n, y, y_stride, bias, stream);
   }
-  if (rows32_pays(w->dev, fmt, m) && !use_gemm(w->dev, fmt, m)) {
+  if (rows32_pays(w->dev, fmt, m, true) && !use_gemm(w->dev, fmt, m)) {
     // Q8_0 / Q4_0 decode batches: quantize once, then the MFMA GEMV. The rows go to the
     // region or this stream's workspace; without room, or under capture without a region, the
     // routes below

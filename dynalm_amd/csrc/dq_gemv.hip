@@ -1540,7 +1540,7 @@ static hipError_t gemv_rows(const WeightDev& w, int af, const uint8_t* acts, int
                             const Workspace* ws, hipStream_t s) {
   const int paf = x != nullptr && af < 0 ? (w.dtype == kQ4_K || w.dtype == kQ6_K ? kActQ8_K : kActPer32) : af;
   // rows per pass: 8, 4, 2 or 1, the most whose staged activations fit the LDS
-  const bool rows32 = dbg == nullptr && x == nullptr && rows32_pays(w, paf, m);
+  const bool rows32 = dbg == nullptr && x == nullptr && rows32_pays(w, paf, m, false);
   int pmax = 8;
   while (pmax > 1 && gemv_lds_bytes(w.dtype, paf, pmax, 16, w.nblk, false) > kGemvMaxLds) pmax /= 2;
   for (int64_t r0 = 0; r0 < m;) {

@@ -178,9 +178,9 @@ bool gemm_b32_supported(int dtype, int af);
 // The MFMA GEMV of Q8_0 / Q4_0 weights x per-32 ActBlockQ8 rows (arb bytes apart) for up to
 // kRows32Max rows (dq_rows32.hip). No workspace.
 constexpr int64_t kRows32Max = 16;
-// Whether m rows of w (activation format af) run faster there, in passes of 16, than in the
-// VALU GEMV's passes.
-bool rows32_pays(const WeightDev& w, int af, int64_t m);
+// Whether m rows of w (activation format af) run faster there, in passes of 16 (after a quantize
+// launch, if the rows still have to be quantized), than in the VALU GEMV's passes.
+bool rows32_pays(const WeightDev& w, int af, int64_t m, bool quantize);
 hipError_t launch_rows32(const WeightDev& w, const uint8_t* acts, int64_t arb, int64_t m, int64_t n0, int64_t n1,
                          float* y, int64_t ys, const float* bias, hipStream_t s);
 // Skinny MFMA GEMV on pre-quantized rows: Q4_K / Q6_K x Q8_K for 2 <= m <=

@@ -22,8 +22,9 @@
 // here, 32 values at ~8 VALU each in every workgroup, took 19.6 us a call against 15.
 //
 // Work split: a workgroup owns 16 TC weight rows and all of K; TC = 4 (the weight load
-// instructions read 1 KB runs, the activations are prepared once per 64 weight rows) while those
-// workgroups fill the CUs, else 2 or 1. A wave's slices are contiguous in K. Of two short slices
+// instructions read 1 KB runs, the activations are prepared once per 64 weight rows) where
+// narrower ones would need a second round on the CUs, else 2 or 1 (N = 11008 Q8_0 at 8 rows 12.4 us
+// against 15.8 with 32-row workgroups). A wave's slices are contiguous in K. Of two short slices
 // (16 of a whole row) each takes two lane groups, which leaves no lane group idle at a slice's end;
 // one after the other they took 4.1 us instead of 3.3 at K = 1024, N = 4096. The long rows of
 // few row groups (two ranges and more) go slice by slice: a load of four consecutive blocks
@@ -241,7 +242,7 @@ template <int WT>
 hipError_t launch_type(const WeightDev& w, const uint8_t* acts, int64_t stride, int64_t m, int64_t n0, int64_t n1,
                        float* y, int64_t ys, const float* bias, hipStream_t s) {
   const int64_t tiles = w.n_pad / 16, cus = w.cus > 0 ? w.cus : 256;
-  const int tc = tiles >= 3 * cus ? 4 : 2 * tiles >= 3 * cus ? 2 : 1;
+  const int tc = tiles > 2 * cus ? 4 : 2 * tiles >= 3 * cus ? 2 : 1;
 #define DQ_ROWS32(...) launch1<WT, __VA_ARGS__>(w, acts, stride, m, n0, n1, y, ys, bias, s)
   switch (gemv_splits(w, kActPer32)) {
     case 1:
@@ -261,20 +262,26 @@ hipError_t launch_type(const WeightDev& w, const uint8_t* acts, int64_t stride, 
 
 }  // namespace
 
-// Against the VALU GEMV's passes of up to 8 rows (quantize + this kernel / fused VALU GEMV), us,
-// K = 4096 unless said: N = 14336 (64-row workgroups) Q4_0 at 4 / 5 / 8 / 12 rows 14.3 / 14.5 /
-// 14.9 / 14.8 against 12.8 / 20.4 / 20.0 / 30.6, Q8_0 18.3 / 18.5 / 18.8 / 19.2 against 15.4 /
-// 27.3 / 20.4 / 34.0; N = 4096 at 2 / 3 / 8 / 12 rows Q4_0 8.3 / 8.3 / 8.8 / 9.2 against 7.8 /
-// 9.5 / 18.0 / 28.2, Q8_0 8.4 / 8.5 / 9.5 / 10.2 against 9.4 / 10.4 / 17.2 / 27.9; N = 4096, K =
-// 14336 at 3 / 8 / 12 rows Q8_0 18.3 / 20.6 / 23.1 against 22.3 / 49.5 / 73.1. (From 13 rows the
-// calls that may take the block GEMM do: it gives the reference's block order bit for bit.)
-bool rows32_pays(const WeightDev& w, int af, int64_t m) {
+// Against the VALU GEMV's passes of up to 8 rows, measured for K = 64 .. 14336, N = 256 .. 32000 (us).
+//  - Rows to quantize first (a launch more; a call from Python, K = 4096): 5 rows and more always
+//    (the VALU GEMV then takes a second pass; its one pass of 8 rows wins below K = 256): N = 4096
+//    Q4_0 at 3 / 4 / 5 / 8 / 12 rows 10.4 / 8.1 / 8.2 / 8.2 / 8.7 against 8.2 / 9.9 / 14.4 / 16.6 /
+//    26.1, K = 1024 at 3 / 4 / 5 / 8 rows 10.4 / 10.4 / 7.7 / 7.7 against 5.3 / 6.3 / 9.6 / 10.0; N =
+//    11008 Q8_0 at 4 / 5 / 8 rows 15.7 / 13.9 / 14.3 against 11.0 / 18.9 / 17.2. At 4 rows only K
+//    >= 4096 pays, on workgroups of at most two tiles (K = 14336, N = 4096 Q8_0 18.9 against 21.5).
+//  - Quantized rows (dq_gemv, GPU time): also 3 and 4 rows of those weights, 3 not on the longest rows:
+//    K = N = 4096 Q4_0 6.0 / 5.8 against 7.0 / 8.3; K = 14336, N = 3072 Q4_0 at 3 rows 15.3 against
+//    12.8; N = 14336 at 4 rows 10.7 against 9.6.
+// (From 13 rows the calls that may take the block GEMM do.)
+bool rows32_pays(const WeightDev& w, int af, int64_t m, bool quantize) {
   if ((w.dtype != kQ8_0 && w.dtype != kQ4_0) || af != kActPer32 ||
       w.n_pad * w.nblk * plane_unit(w.dtype, 0) >= (int64_t)kNoLoad) {
     return false;
   }
-  const bool wide = w.n_pad / 16 >= 3 * (w.cus > 0 ? w.cus : 256);
-  return m >= (wide ? 5 : 3);
+  const bool wide = w.n_pad / 16 > 2 * (w.cus > 0 ? w.cus : 256);
+  if (m >= 5) return m > 8 || w.k >= 256 || !(wide || (quantize && m == 8));
+  if (wide) return false;
+  return quantize ? m == 4 && w.k >= 4096 : m == 4 || (m == 3 && w.k <= 8192);
 }
 
 hipError_t launch_rows32(const WeightDev& w, const uint8_t* acts, int64_t arb, int64_t m, int64_t n0, int64_t n1,

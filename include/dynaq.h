@@ -221,7 +221,7 @@ DQ_API int dq_gemm(const dq_weight* w, int fmt, const void* acts, int64_t m, int
 
 /* y = x . w^T (+ bias): quantize x with dq_act_format_for(w), then GEMV or GEMM by
  * m (Q4_K: GEMM above DQ_GEMV_MAX_ROWS, or above 48 rows for weights of <= 4096 rows;
- * Q8_0 / Q4_0: quantize + the MFMA GEMV from 3 or 5 rows by shape, GEMM from 13 rows; Q6_K: GEMM
+ * Q8_0 / Q4_0: quantize + the MFMA GEMV from 4 or 5 rows by shape, GEMM from 13 rows; Q6_K: GEMM
  * above 64 rows, or above 16 for weights of >= 4096 rows or long K, except long rows on
  * weights of few rows, which run the 16-row skinny GEMV per 16 rows). Every K-quant
  * route gives the same bits; so do the Q8_0 / Q4_0 GEMVs (up to 12 rows, whichever rows are beside
