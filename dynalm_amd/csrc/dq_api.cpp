@@ -149,9 +149,9 @@ struct StreamWs {
 std::mutex g_sws_mu;
 std::vector<StreamWs> g_sws;
 
-template <class F>
-int with_stream_ws(int device, void* stream, size_t need, F&& fn) {
-  std::lock_guard<std::mutex> lock(g_sws_mu);
+// The stream's buffer of at least `need` bytes, under g_sws_mu; where it fails, the call that did
+// is in *what.
+hipError_t stream_ws(int device, void* stream, size_t need, uint8_t** out, const char** what) {
   StreamWs* e = nullptr;
   for (StreamWs& x : g_sws)
     if (x.device == device && x.stream == stream) e = &x;
@@ -161,18 +161,36 @@ int with_stream_ws(int device, void* stream, size_t need, F&& fn) {
   }
   if (e->bytes < need) {
     dq::DeviceScope ds(device);
-    DQ_HIP(ds.err, "hipSetDevice");
+    *what = "hipSetDevice";
+    if (ds.err != hipSuccess) return ds.err;
+    hipError_t rc = hipSuccess;
     if (e->p != nullptr) {
-      DQ_HIP(hipStreamSynchronize(as_stream(stream)), "hipStreamSynchronize");
-      DQ_HIP(hipFree(e->p), "hipFree");
+      *what = "hipStreamSynchronize";
+      if ((rc = hipStreamSynchronize(as_stream(stream))) != hipSuccess) return rc;
+      *what = "hipFree";
+      if ((rc = hipFree(e->p)) != hipSuccess) return rc;
       e->p = nullptr;
       e->bytes = 0;
     }
     const size_t sz = need < (1u << 20) ? (1u << 20) : need;
-    DQ_HIP(hipMalloc(&e->p, sz), "hipMalloc(stream workspace)");
+    *what = "hipMalloc(stream workspace)";
+    if ((rc = hipMalloc(&e->p, sz)) != hipSuccess) {
+      e->p = nullptr;
+      return rc;
+    }
     e->bytes = sz;
   }
-  return fn(static_cast<uint8_t*>(e->p));
+  *out = static_cast<uint8_t*>(e->p);
+  return hipSuccess;
+}
+
+template <class F>
+int with_stream_ws(int device, void* stream, size_t need, F&& fn) {
+  std::lock_guard<std::mutex> lock(g_sws_mu);
+  uint8_t* p = nullptr;
+  const char* what = "";
+  DQ_HIP(stream_ws(device, stream, need, &p, &what), what);
+  return fn(p);
 }
 
 // Whether the stream is not capturing: a captured launch keeps its buffers' addresses, and a
@@ -507,10 +525,10 @@ int matmul_impl(const dq_weight* w, const float* x, int64_t m, int64_t x_stride,
     return dq_gemv(w, fmt, acts, m, 0, w->dev.n, y, y_stride, bias, stream);
   }
   if (rows32_pays(w->dev, fmt, m, true) && !use_gemm(w->dev, fmt, m)) {
-    // Q8_0 / Q4_0 decode batches: quantize once, then the MFMA GEMV. The rows go to the
-    // region or this stream's workspace; without room, or under capture without a region, the
-    // routes below
-    const int64_t need = m * arb;
+    // Q8_0 / Q4_0 decode batches: quantize once, then the MFMA GEMV. The rows go to the region or
+    // this stream's workspace. Without room there, under capture without a region or where the
+    // workspace cannot be had, the fused GEMV below, which needs none (and gives the same bits)
+    const int64_t need = m * arb;  // at most 12 rows (use_gemm)
     auto run = [&](uint8_t* p) -> int {
       DQ_HIP(launch_quantize(fmt, x, m, w->dev.k, m > 1 ? x_stride : w->dev.k, p, arb, s), "quantize launch");
       DQ_HIP(launch_gemv(w->dev, fmt, p, arb, m, 0, w->dev.n, y, y_stride, bias, nullptr, s), "gemv launch");
@@ -518,8 +536,12 @@ int matmul_impl(const dq_weight* w, const float* x, int64_t m, int64_t x_stride,
     };
     if (r.base != nullptr) {
       if ((size_t)need <= r.bytes) return run(r.base);
-    } else if (need < ((int64_t)1 << 32) && m <= 65535 && not_capturing(stream)) {
-      return with_stream_ws(w->dev.device, stream, (size_t)need, run);
+    } else if (not_capturing(stream)) {
+      std::lock_guard<std::mutex> lock(g_sws_mu);
+      uint8_t* p = nullptr;
+      const char* what = "";
+      if (stream_ws(w->dev.device, stream, (size_t)need, &p, &what) == hipSuccess) return run(p);
+      (void)hipGetLastError();
     }
   }
   if (!use_gemm(w->dev, fmt, m)) {

@@ -1,0 +1,89 @@
+"""Which route dq_matmul's Q8_0 / Q4_0 decode batches take, on the CPU: the library's HIP calls go to a
+stand-in that allocates host memory, refuses allocations on demand and counts kernel launches
+(quantize + MFMA GEMV: two, the VALU GEMV's single pass: one). No kernel runs."""
+from __future__ import annotations
+
+import os
+import subprocess
+import sys
+
+import pytest
+
+import dynalm_amd as dq
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+FAKE = r"""
+#include <stddef.h>
+#include <stdlib.h>
+#include <string.h>
+int launches, refuse, capturing, relaxed_mallocs;
+static int mode;  /* hipStreamCaptureModeGlobal */
+typedef struct { unsigned x, y, z; } d3;
+int hipGetDevice(int* d) { *d = 0; return 0; }
+int hipSetDevice(int d) { return 0; }
+int hipDeviceGetAttribute(int* v, int a, int d) { *v = 256; return 0; }
+int hipMalloc(void** p, size_t n) {
+  if (refuse) { *p = (void*)16; return 2; }
+  relaxed_mallocs += mode == 2;
+  *p = malloc(n);
+  return 0;
+}
+int hipFree(void* p) { free(p); return 0; }
+int hipMemcpyAsync(void* d, const void* s, size_t n, int k, void* st) { memcpy(d, s, n); return 0; }
+int hipMemsetAsync(void* d, int v, size_t n, void* st) { memset(d, v, n); return 0; }
+int hipStreamSynchronize(void* s) { return 0; }
+int hipDeviceSynchronize(void) { return 0; }
+int hipStreamIsCapturing(void* s, int* c) { *c = capturing; return 0; }
+int hipThreadExchangeStreamCaptureMode(int* m) { int o = mode; mode = *m; *m = o; return 0; }
+int hipFuncSetAttribute(const void* f, int a, int v) { return 0; }
+int hipGetLastError(void) { return 0; }
+int __hipPushCallConfiguration(d3 g, d3 b, size_t l, void* s) { return 0; }
+int __hipPopCallConfiguration(d3* g, d3* b, size_t* l, void** s) { return 0; }
+int hipLaunchKernel(const void* f, d3 g, d3 b, void** a, size_t l, void* s) { ++launches; return 0; }
+"""
+
+CALLS = r"""
+import ctypes, sys
+import numpy as np
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import dynalm_amd as dq
+var = lambda n: ctypes.c_int.in_dll(fake, n)
+STREAM = 0x1000
+def count(w, m, stream=STREAM, **kw):
+    for k, v in kw.items(): var(k).value = v
+    var("launches").value = 0
+    dq.matmul(w, 64, m, w.k, 64, w.n, None, stream)  # (the pointers are never read here)
+    for k in kw: var(k).value = 0
+    return var("launches").value
+def weight(t, n, k):
+    return dq.Weight.upload(t, np.zeros((n, dq.row_bytes(t, k)), np.uint8), k)
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    d = tmp_path_factory.mktemp("fakehip")
+    (d / "f.c").write_text(FAKE)
+    so = str(d / "libfakehip.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-w", "-o", so, str(d / "f.c")], check=True)
+
+    def run(body: str) -> None:
+        r = subprocess.run([sys.executable, "-c", CALLS + body, so], cwd=ROOT, capture_output=True, text=True)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    if not os.path.exists(dq.lib_path()):
+        pytest.skip("the library is not built")
+    return run
+
+
+def test_without_a_workspace(fake):
+    """A refused allocation leaves the call on the GEMV that needs none; a later one gets it."""
+    fake("""
+w = weight(dq.Q4_0, 300, 512)
+assert count(w, 8, refuse=1) == 1
+assert count(w, 8, refuse=1) == 1
+assert count(w, 8) == 2
+assert count(w, 8, refuse=1) == 2  # (it is there now)
+assert count(w, 8, capturing=1) == 1
+""")
