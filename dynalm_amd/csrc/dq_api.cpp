@@ -149,6 +149,17 @@ struct StreamWs {
 std::mutex g_sws_mu;
 std::vector<StreamWs> g_sws;
 
+// This thread's stream-capture mode is "relaxed" for the object's life: an allocation neither fails
+// for nor invalidates a capture that another thread has begun.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  bool ok;
+  RelaxedCapture() : ok(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+  ~RelaxedCapture() {
+    if (ok) (void)hipThreadExchangeStreamCaptureMode(&mode);  // (back to what it was)
+  }
+};
+
 // The stream's buffer of at least `need` bytes, under g_sws_mu; where it fails, the call that did
 // is in *what.
 hipError_t stream_ws(int device, void* stream, size_t need, uint8_t** out, const char** what) {
@@ -163,6 +174,7 @@ hipError_t stream_ws(int device, void* stream, size_t need, uint8_t** out, const
     dq::DeviceScope ds(device);
     *what = "hipSetDevice";
     if (ds.err != hipSuccess) return ds.err;
+    RelaxedCapture relaxed;
     hipError_t rc = hipSuccess;
     if (e->p != nullptr) {
       *what = "hipStreamSynchronize";

@@ -162,6 +162,43 @@ def test_first_call_under_capture(cuda):
         check(O.Q4_0, rows, x, k, host(e))
 
 
+def test_beside_another_threads_capture(cuda):
+    """The first call on a stream (which allocates its workspace) while another thread captures: the
+    call runs and the capture stays valid."""
+    import ctypes
+    import threading
+
+    m, n, k = 8, 300, 512
+    rows = gguf_weights(O.Q4_0, n, k, 6900)
+    w = dq.Weight.upload(O.Q4_0, rows, k)
+    x = activations(m, k, 6901)
+    xd, y, z = dev(x), torch.zeros((m, n), device="cuda"), torch.zeros(8, device="cuda")
+    hip = ctypes.CDLL("libamdhip64.so")
+    fresh = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(fresh)) == 0
+    err = []
+
+    def call():
+        try:
+            dq.matmul(w, xd, m, k, y, n, None, fresh.value)
+        except Exception as e:  # noqa: BLE001
+            err.append(e)
+
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        z.fill_(1.0)
+        t = threading.Thread(target=call)
+        t.start()
+        t.join()
+    assert not err
+    assert hip.hipStreamSynchronize(fresh) == 0
+    check(O.Q4_0, rows, x, k, host(y))
+    g.replay()
+    assert host(z).all()
+    assert hip.hipStreamDestroy(fresh) == 0
+
+
 @pytest.mark.parametrize("t", TYPES32, ids=lambda t: O.TYPE_NAMES[t])
 def test_capture_outlives_the_stream_workspace(cuda, t):
     """A call captured on a stream that has a workspace does not use it: the graph replays

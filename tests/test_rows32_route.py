@@ -87,3 +87,15 @@ assert count(w, 8) == 2
 assert count(w, 8, refuse=1) == 2  # (it is there now)
 assert count(w, 8, capturing=1) == 1
 """)
+
+
+def test_allocates_in_relaxed_capture_mode(fake):
+    """Another thread's capture is neither an obstacle to the allocation nor invalidated by it."""
+    fake("""
+w = weight(dq.Q4_0, 300, 512)
+before = var("relaxed_mallocs").value
+assert count(w, 8) == 2 and var("relaxed_mallocs").value == before + 1
+m = ctypes.c_int(0)
+fake.hipThreadExchangeStreamCaptureMode(ctypes.byref(m))
+assert m.value == 0
+""")
