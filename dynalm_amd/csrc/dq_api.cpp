@@ -538,8 +538,9 @@ int matmul_impl(const dq_weight* w, const float* x, int64_t m, int64_t x_stride,
   }
   if (rows32_pays(w->dev, fmt, m, true) && !use_gemm(w->dev, fmt, m)) {
     // Q8_0 / Q4_0 decode batches: quantize once, then the MFMA GEMV. The rows go to the region or
-    // this stream's workspace. Without room there, under capture without a region or where the
-    // workspace cannot be had, the fused GEMV below, which needs none (and gives the same bits)
+    // this stream's workspace. Without room there, under capture without a region, on the
+    // per-thread default stream (one handle for every thread's own stream) or where the workspace
+    // cannot be had, the fused GEMV below, which needs none (and gives the same bits)
     const int64_t need = m * arb;  // at most 12 rows (use_gemm)
     auto run = [&](uint8_t* p) -> int {
       DQ_HIP(launch_quantize(fmt, x, m, w->dev.k, m > 1 ? x_stride : w->dev.k, p, arb, s), "quantize launch");
@@ -548,7 +549,7 @@ int matmul_impl(const dq_weight* w, const float* x, int64_t m, int64_t x_stride,
     };
     if (r.base != nullptr) {
       if ((size_t)need <= r.bytes) return run(r.base);
-    } else if (not_capturing(stream)) {
+    } else if (s != hipStreamPerThread && not_capturing(stream)) {
       std::lock_guard<std::mutex> lock(g_sws_mu);
       uint8_t* p = nullptr;
       const char* what = "";

@@ -162,6 +162,40 @@ def test_first_call_under_capture(cuda):
         check(O.Q4_0, rows, x, k, host(e))
 
 
+def test_threads_on_the_per_thread_default_stream(cuda):
+    """Threads that each pass hipStreamPerThread (handle 2) at once have their own rows' outputs."""
+    import ctypes
+    import threading
+
+    m, n, k = 8, 2000, 1024
+    rows = gguf_weights(O.Q4_0, n, k, 6950)
+    w = dq.Weight.upload(O.Q4_0, rows, k)
+    hip = ctypes.CDLL("libamdhip64.so")
+    xs = [dev(activations(m, k, 6951 + i)) for i in range(4)]
+    ys = [[torch.zeros((m, n), device="cuda") for _ in range(50)] for _ in xs]
+    want = []
+    for x in xs:
+        y = torch.zeros((m, n), device="cuda")
+        dq.matmul(w, x, m, k, y, n, None, torch.cuda.current_stream().cuda_stream)
+        want.append(host(y).copy())
+    rc = []
+
+    def calls(i):
+        for y in ys[i]:
+            dq.matmul(w, xs[i], m, k, y, n, None, 2)
+        rc.append(hip.hipStreamSynchronize(ctypes.c_void_p(2)))
+
+    threads = [threading.Thread(target=calls, args=(i,)) for i in range(len(xs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert rc == [0] * len(xs)
+    for i, y in enumerate(ys):
+        for z in y:
+            assert np.array_equal(host(z), want[i])
+
+
 def test_beside_another_threads_capture(cuda):
     """The first call on a stream (which allocates its workspace) while another thread captures: the
     call runs and the capture stays valid."""

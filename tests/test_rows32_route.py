@@ -89,6 +89,16 @@ assert count(w, 8, capturing=1) == 1
 """)
 
 
+def test_per_thread_default_stream(fake):
+    """hipStreamPerThread is one handle for a stream of each thread's own: no buffer is kept for it."""
+    fake("""
+w = weight(dq.Q8_0, 300, 512)
+assert count(w, 8, stream=2) == 1
+assert count(w, 8) == 2 and count(w, 8, stream=0) == 2
+assert count(w, 8, stream=2) == 1
+""")
+
+
 def test_allocates_in_relaxed_capture_mode(fake):
     """Another thread's capture is neither an obstacle to the allocation nor invalidated by it."""
     fake("""
