@@ -109,3 +109,15 @@ m = ctypes.c_int(0)
 fake.hipThreadExchangeStreamCaptureMode(ctypes.byref(m))
 assert m.value == 0
 """)
+
+
+def test_where_two_launches_pay(fake):
+    """Short rows and few of them stay on one launch of the VALU GEMV (rows32_pays)."""
+    fake("""
+for t in (dq.Q8_0, dq.Q4_0):
+    for n, k, rows in ((300, 512, {2: 1, 3: 1, 4: 1, 5: 2, 7: 2, 8: 2, 12: 2}), (300, 128, {3: 1, 8: 1, 9: 2}),
+                       (4096, 4096, {3: 1, 4: 2}), (11008, 4096, {3: 1, 4: 1, 5: 2, 8: 2})):
+        w = weight(t, n, k)
+        for m, want in rows.items():
+            assert count(w, m) == want, (n, k, m)
+""")
