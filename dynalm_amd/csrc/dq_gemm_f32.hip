@@ -9,9 +9,9 @@
 //   Q8_0  (float)q * d,  Q4_0  (float)(nibble - 8) * d
 // i.e. an integer code, which bf16 holds exactly, times a scale that all 32 (Q6_K: 16)
 // values of a block share. The products therefore run on the bf16 matrix cores, 16 times
-// the rate of v_mfma_f32: each fp32 activation splits exactly into three bf16 parts
-// (8 + 8 + 8 significand bits, round to nearest), x = hi + mid + lo, and one block's
-//   S = sum_k x_k q_k
+// the rate of v_mfma_f32: each fp32 activation times 2^24 splits exactly into three bf16 parts
+// (8 + 8 + 8 significand bits, round to nearest), 2^24 x = hi + mid + lo, and one block's
+//   S = sum_k 2^24 x_k q_k
 // is three bf16 MFMAs per K-step into one fp32 accumulator. Every product is exact (8 x at
 // most 8 bits), so S has fp32 rounding only, and acc = fma(scale, S, acc) applies the
 // scale once per block. Q4_K's offsets are Mn = sum_j m_j X_j, X_j the block's fp32
@@ -20,17 +20,21 @@
 // bits), so a one-hot row returns the expanded weight bit for bit, in whichever order the
 // two are added. Error against the exact product at K = 4096 (N(0, 1)-like rows): 2-norm
 // relative 2.9e-7, against 1.1e-6 for v_mfma_f32_32x32x2_f32 over expanded weights (2048
-// dependent fp32 additions per output; here 128 plus the sums inside an MFMA).
+// dependent fp32 additions per output; here 128 plus the sums inside an MFMA). The 2^24, taken off
+// the finished sum, keeps the parts of every fp32 value, subnormal ones too, in bf16's normal range
+// (unscaled, rows near 1e-36 came out 2e-5 off and near 1e-39 2e-2); it costs one of the split's 6.5
+// VALU per value (K = 4096, N = 14336, M = 512: 174.7 -> 175.3 us, N = 4096, M = 16: 62.6 -> 65.3).
 //
 // Work split: a workgroup has 8 waves over 32 RG activation rows x 32 NTW (4 / RG) weight
 // rows. Waves w and w + 4 (one SIMD) hold the same output tiles and take the two 32-value
 // blocks of each 64-value chunk; their sums are added at the end, so an output's order of
 // additions depends on K alone, not on the tile shape, the row count or the row. A wave
-// splits its own 32 rows' activations (5.5 VALU per value) for NTW tiles, through LDS that no
+// splits its own 32 rows' activations (6.5 VALU per value) for NTW tiles, through LDS that no
 // other wave touches; the weight codes become bf16 once per workgroup, in two LDS buffers.
 // The split in the kernel keeps the call free of workspaces, launches and library state.
 //
-// Non-finite inputs: an infinity has no exact split (its mid part is inf - inf), so
+// Non-finite and huge inputs: an infinity has no exact split (its mid part is inf - inf) and 2^24 x
+// overflows from 2^104 (2e31) on, so
 // outputs that come out infinite or NaN are recomputed as plain fp32 dot products of the
 // expanded weights in index order, which gives what IEEE arithmetic gives there.
 //
@@ -58,11 +62,13 @@ namespace dq {
 namespace {
 
 typedef float v2f_t __attribute__((ext_vector_type(2)));
+typedef float v4f_t __attribute__((ext_vector_type(4)));
 typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
 typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
 
 constexpr int kKc = 32;               // K values per block: a block (Q8_0, Q4_0) or sub-block (K-quants)
 constexpr int kThreadsF = 512;
+constexpr float kXScale = 0x1p24f;    // of the activations (see the split above)
 constexpr u32 kNoLoad = 0xFFFFFFF0u;  // a buffer offset past every resource: the load returns zeros
 
 DQ_DEV v16f_t mfma_bf(v4u a, v4u b, v16f_t c) {
@@ -390,12 +396,14 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
       xop + ((lane >> 2) & 1) * kXs + ((lane >> 1) & 1) * 640 + (lane >> 3) * 16 + (lane & 1) * 8;
   float xsum[4] = {0, 0, 0, 0};
   auto split_x = [&](int set, int i) {
-    const v4u v = xv[set][i];
+    v4f_t v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = as_f(xv[set][i][j]) * kXScale;
     v2u hi, mid, lo;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       u32 h, md, l;
-      split3(as_f(v[2 * j]), as_f(v[2 * j + 1]), h, md, l);
+      split3(v[2 * j], v[2 * j + 1], h, md, l);
       hi[j] = h;
       mid[j] = md;
       lo[j] = l;
@@ -403,7 +411,7 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
     *reinterpret_cast<v2u*>(x_wr + 128 * i) = hi;
     *reinterpret_cast<v2u*>(x_wr + 128 * i + kXblk) = mid;
     *reinterpret_cast<v2u*>(x_wr + 128 * i + 2 * kXblk) = lo;
-    if constexpr (WT == kQ4_K) xsum[i] = red8f((as_f(v.x) + as_f(v.y)) + (as_f(v.z) + as_f(v.w)));
+    if constexpr (WT == kQ4_K) xsum[i] = red8f((v.x + v.y) + (v.z + v.w));
   };
   // Q4_K: the block's X_j as three bf16 (lane l the row 8 (l % 4) + l / 8) into slot c % 4 of
   // the super-block's operand: lane r hi (bytes 0..7) and mid (8..15), lane 32 + r lo and 0
@@ -646,7 +654,7 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int r = 4 * q + e, row = 32 * rg + 8 * q + 4 * lg + e;
-            const float v = acc[n][r] + as_f(o[e]);
+            const float v = (acc[n][r] + as_f(o[e])) * (1.0f / kXScale);
             if (in && row < mrows) {
               bad |= !(fabsf(v) <= 3.40282347e38f);
               y[(mbase + row) * ys + nn] = bias ? v + bv : v;

@@ -76,3 +76,17 @@ def test_non_finite_and_extreme_rows(cuda, t):
     clean = activations(m, k, 4401)
     same = [r for r in range(m) if r not in odd + [11, 13]]
     assert np.array_equal(run(t, rows, clean, k)[same].view(np.uint32), y[same].view(np.uint32))
+
+
+@pytest.mark.parametrize("t", TYPES, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("m,n", [(20, 100), (130, 700)])
+def test_rows_of_every_magnitude(cuda, t, m, n):
+    """Rows from subnormal values up keep fp32's relative error: the split holds every fp32 value."""
+    k = 1024
+    rows = gguf_weights(t, n, k, 4500 + t)
+    x = activations(m, k, 4501).astype(np.float64)
+    x = (x * 10.0 ** np.linspace(-42, 34, m)[:, None]).astype(np.float32)
+    x[3, ::2] = 0.0
+    want, mag = exact(t, rows, x, k)
+    # the class's rounding, and half of the subnormal step where the output falls below the normal range
+    assert np.all(np.abs(run(t, rows, x, k) - want) <= 2e-6 * mag + 2.0**-150)
