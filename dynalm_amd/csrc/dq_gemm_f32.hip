@@ -34,9 +34,10 @@
 // The split in the kernel keeps the call free of workspaces, launches and library state.
 //
 // Non-finite and huge inputs: an infinity has no exact split (its mid part is inf - inf) and 2^24 x
-// overflows from 2^104 (2e31) on, so
-// outputs that come out infinite or NaN are recomputed as plain fp32 dot products of the
-// expanded weights in index order, which gives what IEEE arithmetic gives there.
+// overflows from 2^104 (2e31) on, so the tiles of outputs that come out infinite or NaN are run
+// again on v_mfma_f32_32x32x2 over expanded weights, and those outputs taken from there. With
+// every row holding a NaN or an infinity M = 512, K = 4096, N = 14336 takes 1110 us
+// (all of it on v_mfma_f32 600; one dot per lane and output, as it was, 33500).
 //
 // Q4_K, K = 4096, N = 14336, M = 512: 543 -> 172 us (111 -> 350 TFLOP/s); Q6_K K = 14336,
 // N = 4096: 1207 -> 290; Q8_0 4096 x 4096: 306 -> 79; M = 16 at N = 14336: 314 -> 72. What
@@ -237,32 +238,38 @@ struct Raw<kQ4_0> {
   }
 };
 
-// One expanded weight value, k of the row at (gb, r): the plain fp32 path.
+// The expanded weights k .. k + 3 (k % 4 == 0) of the row at (gb, r): the plain fp32 path.
 template <int WT>
-DQ_DEV float expand1(const __amdgpu_buffer_rsrc_t* rs, u32 gb, u32 r, u32 k) {
-  auto ld1 = [](__amdgpu_buffer_rsrc_t p, u32 off) -> u32 { return __builtin_amdgcn_raw_buffer_load_b8(p, off, 0, 0); };
+DQ_DEV v4f_t expand4(const __amdgpu_buffer_rsrc_t* rs, u32 gb, u32 r, u32 k) {
+  v4f_t w;
   if constexpr (WT == kQ4_K) {
     const u32 b = gb + k / 256, j = k / 32 % 8, l = k % 32;
     const v4u hd = ld16(rs[1], (b * 64 + r) * 16);
-    const u32 qb = ld1(rs[0], ((b * 8 + 2 * (j >> 1) + l / 16) * 64 + r) * 16 + l % 16) ^ 0x80u;
+    const u32 q = ld4(rs[0], ((b * 8 + 2 * (j >> 1) + l / 16) * 64 + r) * 16 + l % 16) ^ 0x80808080u;
     int sc, mn;
     scale_min_k4((int)j, hd.y, hd.z, hd.w, sc, mn);
-    return fmaf((float)((j & 1) ? qb >> 4 : qb & 15u), h2f(hd.x) * (float)sc, -(h2f(hd.x >> 16) * (float)mn));
+    const float d = h2f(hd.x) * (float)sc, o = -(h2f(hd.x >> 16) * (float)mn);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = fmaf((float)((q >> (8 * e + 4 * (j & 1))) & 15u), d, o);
   } else if constexpr (WT == kQ6_K) {
     const u32 b = gb + k / 256, u = k / 32 % 8, p = u >> 2, s = u & 3, l = k % 32;
-    const u32 ql = ld1(rs[0], ((b * 8 + 4 * p + 2 * (s & 1) + l / 16) * 64 + r) * 16 + l % 16);
-    const u32 qh = ld1(rs[1], ((b * 4 + 2 * p + l / 16) * 64 + r) * 16 + l % 16);
-    const int q = (int)(((ql >> (4 * (s >> 1))) & 15u) | (((qh >> (2 * s)) & 3u) << 4)) - 32;
-    const int sc = (int8_t)ld1(rs[2], (b * 64 + r) * 16 + k / 16 % 16);
-    return (float)q * (h2f(ld2(rs[3], (b * 64 + r) * 2)) * (float)sc);
-  } else if constexpr (WT == kQ8_0) {
-    const u32 b = gb + k / 32, l = k % 32;
-    return (float)(int8_t)ld1(rs[0], ((b * 2 + l / 16) * 64 + r) * 16 + l % 16) * h2f(ld2(rs[1], (b * 64 + r) * 2));
+    const u32 ql = ld4(rs[0], ((b * 8 + 4 * p + 2 * (s & 1) + l / 16) * 64 + r) * 16 + l % 16) >> (4 * (s >> 1));
+    const u32 qh = ld4(rs[1], ((b * 4 + 2 * p + l / 16) * 64 + r) * 16 + l % 16) >> (2 * s);
+    const int sc = (int8_t)__builtin_amdgcn_raw_buffer_load_b8(rs[2], (b * 64 + r) * 16 + k / 16 % 16, 0, 0);
+    const float d = h2f(ld2(rs[3], (b * 64 + r) * 2)) * (float)sc;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      w[e] = (float)((int)(((ql >> (8 * e)) & 15u) | (((qh >> (8 * e)) & 3u) << 4)) - 32) * d;
   } else {
     const u32 b = gb + k / 32, l = k % 32;
-    const u32 qb = ld1(rs[0], (b * 64 + r) * 16 + l % 16);
-    return (float)((int)((l < 16 ? qb : qb >> 4) & 15u) - 8) * h2f(ld2(rs[1], (b * 64 + r) * 2));
+    const float d = h2f(ld2(rs[1], (b * 64 + r) * 2));
+    const u32 q = WT == kQ8_0 ? ld4(rs[0], ((b * 2 + l / 16) * 64 + r) * 16 + l % 16)
+                              : ld4(rs[0], (b * 64 + r) * 16 + l % 16) >> (l < 16 ? 0 : 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      w[e] = (float)(WT == kQ8_0 ? (int)(int8_t)((q >> (8 * e)) & 0xFFu) : (int)((q >> (8 * e)) & 15u) - 8) * d;
   }
+  return w;
 }
 
 // A wave's activation operands: block (s, part) of K-step s at 3904 s + 1280 part, lane
@@ -663,23 +670,35 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
         }
       }
     }
-    // outputs that are infinite or NaN: the plain fp32 dot product in index order
+    // outputs that are infinite or NaN: their tile on v_mfma_f32_32x32x2 over the expanded weights
+    // (lane l supplies row / column l % 32 and K value l / 32 of each pair, here 4 lg + e of eight)
     if (__builtin_expect(__ballot(bad) != 0, 0)) {
-      const int lo = g == 0 ? 0 : T::kHalf, hi = g == 0 ? T::kHalf : NTW;
+      const int64_t xrow = 32 * rg + li < mrows ? 32 * rg + li : mrows - 1;
 #pragma unroll 1
-      for (int e = lo * 16; e < hi * 16; ++e) {
-        const int n = e >> 4, r = e & 15, row = 32 * rg + 8 * (r >> 2) + 4 * lg + (r & 3);
+      for (int n = g == 0 ? 0 : T::kHalf; n < (g == 0 ? T::kHalf : NTW); ++n) {
         const int64_t nn = nbase + 32 * (cg * NTW + n) + li;
-        if (nn < n0 || nn >= n1 || row >= mrows) continue;
-        float* out = y + (mbase + row) * ys + nn;
-        const float old = *out;
-        if (fabsf(old) <= 3.40282347e38f) continue;
-        const float* xr = x + (mbase + row) * xs;
+        const bool in = nn >= n0 && nn < n1;
+        float* out = y + (mbase + 32 * rg + 4 * lg) * ys + nn;
+        u32 redo = 0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int dr = 8 * (r >> 2) + (r & 3);
+          if (in && 32 * rg + 4 * lg + dr < mrows && !(fabsf(out[dr * ys]) <= 3.40282347e38f)) redo |= 1u << r;
+        }
+        if (__ballot(redo != 0) == 0) continue;
         const u32 gb = (u32)((nn >> 6) * nblk), rr = (u32)(nn & 63);
-        float v = 0;
-#pragma unroll 4
-        for (int kk = 0; kk < k; ++kk) v = fmaf(xr[kk], expand1<WT>(rs, gb, rr, (u32)kk), v);
-        *out = bias ? v + bias[nn] : v;
+        v16f_t v{};
+#pragma unroll 2
+        for (int kk = 0; kk < k; kk += 8) {
+          const v4u xq = ld16(rx, (u32)((xrow * xs + kk + 4 * lg) * 4));
+          const v4f_t wq = expand4<WT>(rs, gb, rr, (u32)(kk + 4 * lg));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v = __builtin_amdgcn_mfma_f32_32x32x2f32(as_f(xq[e]), wq[e], v, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          if ((redo >> r) & 1u) out[(8 * (r >> 2) + (r & 3)) * ys] = bias ? v[r] + bias[nn] : v[r];
+        }
       }
     }
   }

@@ -79,6 +79,31 @@ def test_non_finite_and_extreme_rows(cuda, t):
 
 
 @pytest.mark.parametrize("t", TYPES, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("m,n,blocks", SHAPES)
+def test_many_odd_rows(cuda, t, m, n, blocks):
+    """Batches whose rows hold infinities, NaN and values past the split's range, at the edges of every
+    tile shape: IEEE's result in each, with a bias, beside rows that keep their bits."""
+    k = 256 * max(1, blocks // 4) if t in (O.Q4_K, O.Q6_K) else 32 * blocks
+    rows = gguf_weights(t, min(n, 300), k, 4600 + t + m)
+    rows = np.tile(rows, (-(-n // rows.shape[0]), 1))[:n].copy()
+    x = activations(m, k, 4700 + m)
+    bias = O.normal(4800 + m, n)
+    clean = run(t, rows, x, k, bias)
+    x[::4, k - 1] = np.inf
+    x[1::4, k // 2] = np.nan
+    x[2::4, 0] = np.float32(-2e35)
+    y = run(t, rows, x, k, bias)
+    want, mag = exact(t, rows, x, k)
+    want += bias
+    fin = np.isfinite(want)
+    with np.errstate(invalid="ignore"):
+        diff = np.abs(y - want)
+    assert np.array_equal(np.isfinite(y), fin) and np.array_equal(y[~fin], want[~fin].astype(np.float32), equal_nan=True)
+    assert np.all(diff[fin] <= (2e-6 * (mag + np.abs(bias)))[fin])
+    assert np.array_equal(y[3::4].view(np.uint32), clean[3::4].view(np.uint32))
+
+
+@pytest.mark.parametrize("t", TYPES, ids=lambda t: O.TYPE_NAMES[t])
 @pytest.mark.parametrize("m,n", [(20, 100), (130, 700)])
 def test_rows_of_every_magnitude(cuda, t, m, n):
     """Rows from subnormal values up keep fp32's relative error: the split holds every fp32 value."""
