@@ -366,9 +366,9 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
 #pragma unroll
     for (int p = 0; p < T::kPasses; ++p) raw[set][p].load(rs, egb[p], nblk, c, esel[p], er[p]);
   };
-  auto put_w = [&](int c, int set, auto part) {
+  auto put_w = [&](int c, int dst, int set, auto part) {  // chunk c's bytes, into chunk dst's buffer
     if (!conv) return;
-    uint8_t* buf = smem + (c & 1) * T::kBuf;
+    uint8_t* buf = smem + (dst & 1) * T::kBuf;
 #pragma unroll
     for (int p = 0; p < T::kPasses; ++p) {
       const int row = erow[p];
@@ -477,8 +477,8 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
 #pragma unroll
     for (int i = 0; i < 4; ++i) load_x(clamp(d), d, i);
   }
-  put_w(0, 0, P0{});
-  put_w(0, 0, P1{});
+  put_w(0, 0, 0, P0{});
+  put_w(0, 0, 0, P1{});
   keep_hd(0);
   put_mins(0);
 #pragma unroll
@@ -522,9 +522,9 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
   auto chunk = [&](int c, int set) {
     const uint8_t* buf = smem + (c & 1) * T::kBuf;
     const uint8_t* nbuf = smem + ((c + 1) & 1) * T::kBuf;
-    // chunk c + 1 (clamped: the last iteration redoes the last chunk into the buffer no one
-    // reads again) is converted between the MFMAs of chunk c; its registers are reloaded for
-    // chunk c + 1 + kDepth as soon as they are read
+    // chunk c + 1 (past the end: the last chunk's bytes again, still into the buffer, mins and
+    // offsets of c + 1, which no one reads then) is converted between the MFMAs of chunk c; its
+    // registers are reloaded for chunk c + 1 + kDepth as soon as they are read
     const int cn = clamp(c + 1), cl = clamp(c + 1 + T::kDepth);
 #pragma unroll
     for (int n = 0; n < NTW; ++n) {
@@ -556,9 +556,9 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
 #pragma unroll
       for (int q = 0; q < 6; ++q) {
         if (q * (kLast > 0 ? kLast : 1) / 6 != n) continue;
-        if (q == 0) put_w(cn, set, P0{});
+        if (q == 0) put_w(cn, c + 1, set, P0{});
         if (q == 1) {
-          put_w(cn, set, P1{});
+          put_w(cn, c + 1, set, P1{});
           keep_hd(set);
           load_w(cl, set);
         }
@@ -566,7 +566,7 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
           split_x(set, q - 2);
           load_x(cl, set, q - 2);
         }
-        if (q == 5) put_xsum(cn);
+        if (q == 5) put_xsum(c + 1);
       }
       if (n == kLast && NTW > 1) {
 #pragma unroll
@@ -609,7 +609,7 @@ __global__ __launch_bounds__(kThreadsF) __attribute__((amdgpu_waves_per_eu(2, 2)
         const uint8_t* mins = smem + T::kOffMins + ((c >> 2) & 1) * T::kMins;
         const float* dm = reinterpret_cast<const float*>(mins + 16 * T::kRows) + cg * NTW * 32 + li;
         const uint8_t* mb = mins + (g * T::kRows + cg * NTW * 32 + li) * 8;
-        put_mins(cn >> 2);
+        put_mins((c + 1) >> 2);
         const v4u xm = lds16(xmop + ((c >> 2) & 1) * 1024 + lane * 16);
         fold(kLastTile);  // before its offsets, as the other tiles' sums
         fp0 = 0;
