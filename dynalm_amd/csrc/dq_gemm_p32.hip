@@ -14,7 +14,9 @@
 //   per sub-block:    T = fma(da_j, sc_j P_j 2^-24, T)      (one VALU operation per output)
 //   per super-block:  acc = fma(d 2^24, T, acc)             (one per output), T = 0
 // and the mins term Mn = sum_j m_j c_j on two v_mfma_f32_32x32x16_bf16 per super-block (m_j
-// < 64 is exact in bf16; c_j is the exact sum of three bf16 parts), acc = fma(-dmin, Mn, acc).
+// < 64 is exact in bf16; c_j is the exact sum of four scaled bf16 parts, and the weight operands m_j
+// carry the parts' scales and a 2^-9 that keeps Mn, at most 504 times the largest c_j, finite before
+// dmin comes to it), acc = fma(-dmin 2^9, Mn 2^-9, acc).
 // Every product is exact or rounded once, but d multiplies the super-block's sum
 // rather than each term, and the summation order is not qmm's (nor the per-32
 // GEMV's, kernels_generic.cpp:261-279): the outputs agree within the fp32 tolerance of
@@ -44,8 +46,8 @@
 //          hh = l / 32; K-step k = 2 j + h holds values 32 j + 16 hh + 8 h + {0, 2, 1,
 //          3, 4, 6, 5, 7} of the super-block (sub-block j only)
 //   da     [T][nb][j (8)][32 rows] floats
-//   c      [T][nb][part (2)][lane (64)][8 bf16]: row l % 32's eight c_j 2^-9; part 0 hi (lanes
-//          0-31) and mid, part 1 lo and zeros
+//   c      [T][nb][part (2)][lane (64)][8 bf16]: row l % 32's eight c_j; part 0 p0 (lanes 0-31)
+//          and p1, part 1 p2 and p3 (put_c)
 // The K order is the one in which a lane's B operand comes out of two dwords of its
 // weight row's nibbles: values 32 j + t of sub-block j are the low (j even) or high
 // (j odd) nibbles of qs bytes 32 (j / 2) + t (quant_formats.cpp:150-167), so K-step
@@ -89,22 +91,34 @@ DQ_DEV u32 bf_pair(float a, float b) {
   typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
   return __builtin_bit_cast(u32, __builtin_convertvector(v2f_t{a, b}, v2bf_t));
 }
-// c of one (row, sub-block j) into the mins operands of its tile and super-block at cb, times
-// 2^-9 so that sum_j m_j c_j (at most 504 times the largest) stays finite before dmin comes to
-// it: hi + mid + lo exactly in bf16; part 0 holds hi (lanes 0-31) and mid (32-63), part 1 lo and
-// zeros, each lane its row's eight sub-blocks.
+// c of one (row, sub-block j) into the mins operands of its tile and super-block at cb: c = p0 + 2^-7
+// p1 + 2^-15 p2 + 2^-22 p3 in bf16, part 0 holding p0 (lanes 0-31) and p1 (32-63), part 1 p2 and
+// p3, each lane its row's eight sub-blocks. The later parts are scaled up by what they are smaller
+// than c, so that they stay in range for the largest c and hold every bit of the smallest (bf16's
+// subnormal step is 2^-133; p3 is zero unless c is below about 2^-110).
 DQ_DEV void put_c(uint8_t* cb, int r, int j, float c) {
-  c *= 0x1p-9f;
-  // hi truncated, so that a finite c stays finite; an infinite or NaN c is hi alone
-  const u32 hi = as_u(c) & 0xFFFF0000u;
-  const float c1 = fabsf(c) <= 3.40282347e38f ? c - as_f(hi) : 0.0f;
-  const u32 mid = bf_pair(c1, 0.0f);
-  const u32 lo = bf_pair(c1 - as_f(mid << 16), 0.0f);
+  // p0 truncated, so that a finite c stays finite; an infinite or NaN c is p0 alone
+  const u32 p0 = as_u(c) & 0xFFFF0000u;
+  const float c1 = fabsf(c) <= 3.40282347e38f ? (c - as_f(p0)) * 0x1p7f : 0.0f;
+  const u32 p1 = bf_pair(c1, 0.0f);
+  const float c2 = (c1 - as_f(p1 << 16)) * 0x1p8f;
+  const u32 p2 = bf_pair(c2, 0.0f);
+  const u32 p3 = bf_pair((c2 - as_f(p2 << 16)) * 0x1p7f, 0.0f);
   uint16_t* o = reinterpret_cast<uint16_t*>(cb + r * 16) + j;
-  o[0] = (uint16_t)(hi >> 16 | (c != c ? 1u : 0u));  // a NaN whose high bits are an infinity's
-  o[256] = (uint16_t)mid;
-  o[512] = (uint16_t)lo;
-  o[768] = 0;
+  o[0] = (uint16_t)(p0 >> 16 | (c != c ? 1u : 0u));  // a NaN whose high bits are an infinity's
+  o[256] = (uint16_t)p1;
+  o[512] = (uint16_t)p2;
+  o[768] = (uint16_t)p3;
+}
+// bf16 pairs, zero or at least 2^n in magnitude and positive, times 2^-n: the exponent less n,
+// zeros kept by the saturation.
+DQ_DEV v4u bf_scale_down(v4u v, u32 n) {
+  typedef uint16_t v2s __attribute__((ext_vector_type(2)));
+  const v2s e = __builtin_bit_cast(v2s, n * 0x00800080u);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    v[i] = __builtin_bit_cast(u32, __builtin_elementwise_sub_sat(__builtin_bit_cast(v2s, (u32)v[i]), e));
+  return v;
 }
 
 }  // namespace
@@ -314,7 +328,7 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
     rd(0, 0);
     v16f_t sp{};
     float dp = 0;
-    v4u mm{};
+    v4u mm0{}, mm1{};
     // the result of step (j, tt): T += da_j sc_j P_j; the mins and then the super-block's sum
     // into acc with -dmin 2^9 and d 2^24 of the lane's 16 weight rows 8 q + 4 hh + e
     auto fold = [&](int j, int tt) {
@@ -347,8 +361,8 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
         S = mfma_h(w[0], b0, v16f_t{});
         S = mfma_h(w[1], b1, S);
       } else {
-        S = mfma_bf(mm, b0, v16f_t{});
-        S = mfma_bf(mm, b1, S);
+        S = mfma_bf(mm0, b0, v16f_t{});
+        S = mfma_bf(mm1, b1, S);
       }
       if (q > 0) fold((q - 1) / TT, (q - 1) % TT);
       // the next sub-block's weight operands (j = 8: the next super-block's first), nib[g] and
@@ -367,11 +381,13 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
         *reinterpret_cast<float*>(rowd + li * 4) = h2f(hdr.x) * 16777216.0f;
         *reinterpret_cast<float*>(rowd + 128 + li * 4) = h2f(hdr.x >> 16) * -512.0f;
       }
-      if (j == 7 && tt == TT - 1) {  // the mins' weight operand: m_j of the lane's row
+      if (j == 7 && tt == TT - 1) {  // the mins' weight operands: m_j of the lane's row, scaled
         const u32 mA = hdr.z & 0x3F3F3F3Fu, mB = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
         auto mf = [](u32 v, int i) { return (float)((v >> (8 * i)) & 0xFFu); };
-        mm = v4u{bf_pair(mf(mA, 0), mf(mA, 1)), bf_pair(mf(mA, 2), mf(mA, 3)), bf_pair(mf(mB, 0), mf(mB, 1)),
-                 bf_pair(mf(mB, 2), mf(mB, 3))};
+        const v4u m = v4u{bf_pair(mf(mA, 0), mf(mA, 1)), bf_pair(mf(mA, 2), mf(mA, 3)), bf_pair(mf(mB, 0), mf(mB, 1)),
+                          bf_pair(mf(mB, 2), mf(mB, 3))};
+        mm0 = bf_scale_down(m, hh ? 16u : 9u);  // p1, p0
+        mm1 = bf_scale_down(mm0, 15u);          // p3, p2
       }
       // the next super-block's 2 TT pieces of this wave, one every fourth step (past the end the
       // last one's again, into the buffer no one reads)
