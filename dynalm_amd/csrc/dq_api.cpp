@@ -1092,8 +1092,7 @@ int dq_matmul_many(const dq_matmul_job* jobs, int64_t n_jobs, void* stream) {
       others.push_back(i);
     }
   }
-  // one-row K-quant jobs of one k: one launch for up to kGemvManyMax (a single one as
-  // dq_matmul runs it)
+  // one-row K-quant jobs of one k: one launch for up to kGemvManyMax, or each as dq_matmul runs it
   while (!ones.empty()) {
     dq::GemvJob batch[dq::kGemvManyMax];
     int n = 0;
@@ -1106,11 +1105,13 @@ int dq_matmul_many(const dq_matmul_job* jobs, int64_t n_jobs, void* stream) {
         rest.push_back(j);
       }
     }
-    if (n > 1) {
+    if (dq::gemv_many_pays(batch, n)) {
       DQ_HIP(dq::launch_gemv_many(batch, n, s), "grouped gemv launch");
     } else {
-      DQ_HIP(dq::launch_gemv_fused(*batch[0].w, batch[0].x, batch[0].xs, 1, batch[0].y, batch[0].ys, batch[0].bias, s),
-             "gemv launch");
+      for (int i = 0; i < n; ++i) {
+        const dq::GemvJob& j = batch[i];
+        DQ_HIP(dq::launch_gemv_fused(*j.w, j.x, j.xs, 1, j.y, j.ys, j.bias, s), "gemv launch");
+      }
     }
     ones.swap(rest);
   }

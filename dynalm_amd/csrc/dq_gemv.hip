@@ -1428,6 +1428,12 @@ static hipError_t gemv_early(const WeightDev& w, const uint8_t* acts, int64_t ar
   return gemv_launch<WT, AF, M, kFuse, W, 0, kSplit>(w, acts, arb, x, xs, n0, n1, y, ys, bias, dbg, sp, s);
 }
 
+// The Q4_K weights whose one-row GEMV is k_gemv_slab's: 56-row workgroups in one round on the CUs.
+static bool slab_shape(const WeightDev& w) {
+  return w.dtype == kQ4_K && (w.nblk == 8 || w.nblk == 16) &&
+         w.n_pad / kRowGroup * kRowGroup <= (int64_t)kSlabRows * w.cus;
+}
+
 template <int AF, bool kFuse>
 static hipError_t gemv_slab(const WeightDev& w, const uint8_t* acts, const float* x, int64_t n0, int64_t n1, float* y,
                             const float* bias, int32_t* dbg, hipStream_t s) {
@@ -1455,8 +1461,7 @@ static hipError_t gemv_waves(const WeightDev& w, const uint8_t* acts, int64_t ar
   const int64_t groups = w.n_pad / kRowGroup;
   if constexpr (WT == kQ4_K && M == 1 && (AF == kActQ8_K || (AF == kActPer32 && kFuse))) {
     // fewer row groups than CUs: 56-row workgroups spread the row over more CUs
-    if ((w.nblk == 8 || w.nblk == 16) && groups * kRowGroup <= (int64_t)kSlabRows * w.cus &&
-        (AF == kActQ8_K || gemv_splits(w, AF) == 1)) {
+    if (slab_shape(w) && (AF == kActQ8_K || gemv_splits(w, AF) == 1)) {
       return gemv_slab<AF, kFuse>(w, acts, x, n0, n1, y, bias, dbg, s);
     }
   }
@@ -1582,9 +1587,18 @@ static hipError_t many_launch(const OneRowGroup& g, int64_t wgs, size_t lds, hip
   return hipGetLastError();
 }
 
+// Weights of more row groups than CUs stay with launches of their own: those run 8-wave workgroups,
+// two to a CU, where the grouped kernel's 16 waves cost more than the launches (Q4_K N = 32000, K =
+// 1024, two and eight jobs: 16.2 and 59.9 us grouped, 11.2 and 41.7 one by one).
 bool gemv_many_ok(const WeightDev& w) {
-  return (w.dtype == kQ4_K || w.dtype == kQ6_K) && w.nblk <= 64 &&
+  return (w.dtype == kQ4_K || w.dtype == kQ6_K) && w.nblk <= 64 && w.n_pad / kRowGroup <= w.cus &&
          gemv_lds_bytes(w.dtype, kActQ8_K, 1, 16, w.nblk, true) <= kGemvMaxLds;
+}
+
+bool gemv_many_pays(const GemvJob* jobs, int count) {
+  if (count != 2) return count > 2;
+  const int64_t groups = jobs[0].w->n_pad / kRowGroup + jobs[1].w->n_pad / kRowGroup;
+  return groups <= jobs[0].w->cus || !slab_shape(*jobs[0].w) || !slab_shape(*jobs[1].w);
 }
 
 hipError_t launch_gemv_many(const GemvJob* jobs, int count, hipStream_t s) {

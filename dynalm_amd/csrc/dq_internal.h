@@ -227,6 +227,10 @@ hipError_t launch_gemv_mma_many(const GemvJob* jobs, int count, hipStream_t s, c
 // which gemv_many_ok) in one launch, each output with the one-row GEMV's bits.
 constexpr int kGemvManyMax = 8;
 bool gemv_many_ok(const WeightDev& w);
+// Whether one launch is faster than one each: not for a single job, nor for two that fill the CUs in
+// one round each on the 56-row GEMV but not together (N = 9000, K = 2048 / 4096: 9.3 / 11.5 us
+// grouped, 7.6 / 10.4 one by one; three such jobs 9.7 / 12.4 against 10.3 / 14.9).
+bool gemv_many_pays(const GemvJob* jobs, int count);
 hipError_t launch_gemv_many(const GemvJob* jobs, int count, hipStream_t s);
 // Work of one grouped launch of these jobs (<= 8, one nblk) in wave-sized units
 // (workgroups x super-blocks): each unit of a launch on fp32 rows quantizes 16

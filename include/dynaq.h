@@ -273,7 +273,7 @@ typedef struct dq_matmul_job {
 
 /* Several independent matmuls on one stream, e.g. the projections that share one
  * input (Q/K/V, gate/up) or the experts of an MoE layer. One-row K-quant jobs of one k run
- * in one launch for up to 8 of them. The decode-sized K-quant
+ * in one launch for up to 8 of them (weights of no more 64-row groups than CUs). The decode-sized K-quant
  * jobs (Q4_K: 2 <= m <= 16; Q6_K: 2 <= m <= 64) of one k run together in grouped
  * skinny-GEMV launches (up to
  * 8 jobs each, Q4_K and Q6_K mixed) that quantize each job's fp32 rows in the

@@ -121,3 +121,20 @@ for t in (dq.Q8_0, dq.Q4_0):
         for m, want in rows.items():
             assert count(w, m) == want, (n, k, m)
 """)
+
+
+def test_one_row_jobs_grouped(fake):
+    """matmul_many's one-row K-quant jobs share a launch unless their weights fill the CUs alone."""
+    fake("""
+def many(ws):
+    var("launches").value = 0
+    dq.matmul_many([(w, 64, 1, w.k, 64, w.n, None) for w in ws], STREAM)
+    return var("launches").value
+for t in (dq.Q4_K, dq.Q6_K):
+    small, wide = weight(t, 500, 512), weight(t, 256 * 64 + 1, 512)
+    assert many([small] * 3) == 1 and many([weight(t, 256 * 64, 512)] * 8) == 1
+    assert many([wide] * 3) == 3 and many([small, wide, small]) == 2
+slab = weight(dq.Q4_K, 9000, 2048)  # two rounds together, one each on the 56-row GEMV
+assert many([slab] * 2) == 2 and many([slab] * 3) == 1
+assert many([weight(dq.Q4_K, 4096, 2048)] * 2) == 1 and many([weight(dq.Q6_K, 9000, 2048)] * 2) == 1
+""")
