@@ -1680,8 +1680,13 @@ hipError_t launch_gemv(const WeightDev& w, int af, const uint8_t* acts, int64_t 
 }
 
 // (the rows from which dq_matmul_act's int16 GEMMs take over are 5 and 3)
+// Every workgroup quantizes the rows again, so the fused pass loses to a quantize launch once rows
+// x weights are many (graph replay, fused / separate): Q4_K K = 14336, N = 6144 at 2 / 3 / 4 rows 23.0 /
+// 22.7, 29.0 / 27.6, 35.5 / 32.7 us, K = 8192, N = 14336 at 2 rows 21.8 / 21.0, K = 8192, N = 6144 at 4
+// rows 22.4 / 23.2; Q6_K K = 8192, N = 14336 at 2 rows 28.5 / 27.3.
 bool gemv_fuses_q16(const WeightDev& w, int64_t m) {
   if (m < 1 || m > (w.dtype == kQ4_K ? 4 : w.dtype == kQ6_K ? 2 : 0)) return false;
+  if (m > 1 && m * w.n_pad * w.k >= 220000000) return false;
   return gemv_lds_bytes(w.dtype, kActQ16, (int)m, 16, w.nblk, false) <= kGemvMaxLds;
 }
 

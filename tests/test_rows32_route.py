@@ -138,3 +138,18 @@ slab = weight(dq.Q4_K, 9000, 2048)  # two rounds together, one each on the 56-ro
 assert many([slab] * 2) == 2 and many([slab] * 3) == 1
 assert many([weight(dq.Q4_K, 4096, 2048)] * 2) == 1 and many([weight(dq.Q6_K, 9000, 2048)] * 2) == 1
 """)
+
+
+def test_int16_rows_quantized_in_the_gemv(fake):
+    """int16 decode rows are quantized inside the GEMV (one launch less) while rows x weights are few."""
+    fake("""
+def act(w, m):
+    var("launches").value = 0
+    dq.matmul_act(w, dq.ACT_Q16, 64, m, w.k, 64, w.n, None, STREAM)
+    return var("launches").value
+for t, n, k, rows in ((dq.Q4_K, 14336, 512, {1: 1, 4: 1}), (dq.Q6_K, 14336, 512, {1: 1, 2: 1}),
+                      (dq.Q4_K, 6144, 14336, {1: 2, 2: 2, 3: 3, 4: 3}), (dq.Q6_K, 14336, 8192, {1: 1, 2: 2})):
+    w = weight(t, n, k)
+    for m, want in rows.items():
+        assert act(w, m) == want, (n, k, m, act(w, m))
+""")
