@@ -1,6 +1,6 @@
-// dq_f16mma.h -- helpers of the f16-matrix-core GEMMs (dq_gemm_h16.hip,
-// dq_gemm_p32.hip): the 32 x 32 x 16 f16 MFMA, direct-to-LDS buffer loads, LDS reads
-// and the int8 -> f16 operand conversion.
+// dq_f16mma.h -- helpers of the GEMMs on the 16-bit matrix cores (dq_gemm_h16.hip,
+// dq_gemm_p32.hip, dq_gemm_f32.hip): the 32 x 32 x 16 f16 and bf16 MFMAs, direct-to-LDS buffer
+// loads, LDS reads and the conversions to their operands.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -19,6 +19,18 @@ typedef _Float16 v8h_t __attribute__((ext_vector_type(8)));
 DQ_DEV v16f_t mfma_h(v4u a, v4u b, v16f_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h_t, a), __builtin_bit_cast(v8h_t, b), c, 0, 0,
                                                 0);
+}
+typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
+// The same in bf16 (v_mfma_f32_32x32x16_bf16).
+DQ_DEV v16f_t mfma_bf(v4u a, v4u b, v16f_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, a), __builtin_bit_cast(v8bf_t, b), c, 0, 0,
+                                                 0);
+}
+// Two floats as bf16, round to nearest (v_cvt_pk_bf16_f32).
+DQ_DEV u32 bf_pair(float a, float b) {
+  typedef float v2f_t __attribute__((ext_vector_type(2)));
+  typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(u32, __builtin_convertvector(v2f_t{a, b}, v2bf_t));
 }
 DQ_DEV v4u lds16(const uint8_t* p) { return *reinterpret_cast<const v4u*>(p); }
 

@@ -62,24 +62,13 @@ namespace dq {
 
 namespace {
 
-typedef float v2f_t __attribute__((ext_vector_type(2)));
 typedef float v4f_t __attribute__((ext_vector_type(4)));
-typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
-typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
 
 constexpr int kKc = 32;               // K values per block: a block (Q8_0, Q4_0) or sub-block (K-quants)
 constexpr int kThreadsF = 512;
 constexpr float kXScale = 0x1p24f;    // of the activations (see the split above)
 constexpr u32 kNoLoad = 0xFFFFFFF0u;  // a buffer offset past every resource: the load returns zeros
 
-DQ_DEV v16f_t mfma_bf(v4u a, v4u b, v16f_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, a), __builtin_bit_cast(v8bf_t, b), c, 0, 0,
-                                                 0);
-}
-// Two floats as bf16, round to nearest (v_cvt_pk_bf16_f32).
-DQ_DEV u32 bf_pair(float a, float b) {
-  return __builtin_bit_cast(u32, __builtin_convertvector(v2f_t{a, b}, v2bf_t));
-}
 // The exact three-part split of two floats: a pair of bf16 per part.
 DQ_DEV void split3(float a, float b, u32& hi, u32& mid, u32& lo) {
   hi = bf_pair(a, b);

@@ -81,16 +81,6 @@ struct PLds {
 };
 static_assert(PLds<4>::kTotal <= 160 * 1024, "LDS");
 
-typedef __bf16 v8bf_t __attribute__((ext_vector_type(8)));
-DQ_DEV v16f_t mfma_bf(v4u a, v4u b, v16f_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf_t, a), __builtin_bit_cast(v8bf_t, b), c, 0, 0,
-                                                 0);
-}
-DQ_DEV u32 bf_pair(float a, float b) {
-  typedef float v2f_t __attribute__((ext_vector_type(2)));
-  typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(u32, __builtin_convertvector(v2f_t{a, b}, v2bf_t));
-}
 // c of one (row, sub-block j) into the mins operands of its tile and super-block at cb: c = p0 + 2^-7
 // p1 + 2^-15 p2 + 2^-22 p3 in bf16, part 0 holding p0 (lanes 0-31) and p1 (32-63), part 1 p2 and
 // p3, each lane its row's eight sub-blocks. The later parts are scaled up by what they are smaller

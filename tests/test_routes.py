@@ -1,6 +1,6 @@
-"""Which route dq_matmul's Q8_0 / Q4_0 decode batches take, on the CPU: the library's HIP calls go to a
-stand-in that allocates host memory, refuses allocations on demand and counts kernel launches
-(quantize + MFMA GEMV: two, the VALU GEMV's single pass: one). No kernel runs."""
+"""Which routes the decode calls take, on the CPU: the library's HIP calls go to a stand-in that
+allocates host memory, refuses allocations on demand and counts kernel launches (of Q8_0 / Q4_0
+rows: quantize + MFMA GEMV two, the VALU GEMV's single pass one). No kernel runs."""
 from __future__ import annotations
 
 import os
