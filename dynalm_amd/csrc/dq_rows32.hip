@@ -31,8 +31,8 @@
 // touches half the cache lines of four slices' (Q8_0 K = 14336, N = 5120 at 8 rows 30.3 us
 // against 34.2), on 16 waves where one workgroup fills a CU (N = 2048, Q4_0 14.6 against 16.6).
 // What bounds it: Q4_0 K = 4096, N = 14336 at 8 rows takes 10.8 us for 33 MB (3.1 TB/s; the
-// VALU GEMV, which pays its dots for every row, 15.3). A wave's two steps per slice pair are 48
-// MFMAs and ~300 VALU each; loads one or two steps ahead measured alike.
+// VALU GEMV, which pays its dots for every row, 15.3). A wave's four steps are 44 MFMAs (768 clocks)
+// and ~350 VALU (1,400) each; loads one or two steps ahead measured alike.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -117,15 +117,12 @@ __global__ __launch_bounds__(64 * kWaves) void k_rows32(const uint8_t* __restric
   // the lane group's slice of a round, [b, end); its block of step q is b + kB q
   constexpr int kB = 4 / G, kPer = kSplits * WR / kWaves, kRounds = kPer / G;
   static_assert(kPer * kWaves == kSplits * WR && kPer % G == 0, "whole rounds");
-  auto first = [&](int i) {  // the first block of slice i
-    const int sk = i / WR, wl = i % WR, k0 = sk * nblk / kSplits, k1 = (sk + 1) * nblk / kSplits;
-    return k0 + wl * (k1 - k0) / WR;
-  };
   int b, end;
   auto round = [&](int r) {
-    const int i = kPer * wave + G * r + g / kB;
-    b = first(i) + g % kB;
-    end = first(i + 1);
+    const int i = kPer * wave + G * r + g / kB, sk = i / WR, wl = i % WR;
+    const int k0 = sk * nblk / kSplits, k1 = (sk + 1) * nblk / kSplits;
+    b = k0 + wl * (k1 - k0) / WR + g % kB;
+    end = k0 + (wl + 1) * (k1 - k0) / WR;
   };
   round(0);
   v4f_t acc[G][TC];
