@@ -39,12 +39,14 @@
 // every row holding a NaN or an infinity M = 512, K = 4096, N = 14336 takes 1110 us
 // (all of it on v_mfma_f32 600; one dot per lane and output, as it was, 33500).
 //
-// Q4_K, K = 4096, N = 14336, M = 512: 543 -> 172 us (111 -> 350 TFLOP/s); Q6_K K = 14336,
-// N = 4096: 1207 -> 290; Q8_0 4096 x 4096: 306 -> 79; M = 16 at N = 14336: 314 -> 72. What
-// bounds it now: the MFMAs are 81 us of the 172 (117 with operand reads and barriers alone,
-// 123 with the folds), the VALU issue beside them the rest -- removing only the activation
-// split takes 32 us off, the weight conversion 26, the offsets 20, the folds 20 -- 8 VALU per
-// MFMA, where a register-only loop of 2 waves per SIMD hides 4 to 6.
+// Q4_K, K = 4096, N = 14336, M = 512: 543 -> 167-173 us (111 -> 355 TFLOP/s; over weights in turn
+// 214-227, in the same number of clocks at a lower rate); Q6_K K = 14336, N = 4096: 1207 -> 290; Q8_0 4096 x
+// 4096: 306 -> 79; M = 16 at N = 14336: 314 -> 69. What bounds it now: VALU issue beside the MFMAs. A
+// wave's chunk is 44 MFMAs and 364 VALU, 8 per MFMA, where a register-only loop of 2 waves per
+// SIMD hides 4 to 6; the matrix pipe is busy 54% of the clocks and has a VALU op beside it in 55% of
+// those. Timing-only copies (before the scaling): the MFMAs alone 81 us of 172, with operand reads and
+// barriers 117, with the folds too 123; without only the activation split 32 less, the weight
+// conversion 26, the offsets 20, the folds 20.
 //
 // MFMA lane layout (v_mfma_f32_32x32x16_bf16): lane l supplies row (A) / column (B) l % 32
 // and K = 8 (l / 32) .. + 7; result register r of lane l is row 8 (r / 4) + 4 (l / 32) +

@@ -32,12 +32,13 @@
 // tile's two MFMAs. A super-block's operands (128 rows x 256 codes as f16, 64 KB), activation
 // scales and mins operands (4 + 8 KB) go to LDS one interval ahead by direct-to-LDS loads
 // spread over the steps, into a ring of two; one barrier per super-block.
-// What bounds it: issue slots. A wave's super-block is 72 MFMAs and ~870 VALU (the folds 640,
+// What bounds it: issue slots. A wave's super-block is 72 MFMAs and ~910 VALU (the folds 640,
 // the weight operands ~200); two waves per SIMD need 15 clocks of issue per MFMA and 4 per
-// VALU (measured in a register-only loop), 147 K clocks in all at K = 4096, ~65 us. M = 512,
+// VALU (measured in a register-only loop), ~150 K clocks in all at K = 4096, ~66 us. M = 512,
 // N = 14336, kernel alone: 109 -> 96 us; the whole call 112.6 -> 102; M = 77, N = 5003, K =
-// 2304 28.8 -> 25.9. Without its loads 109 of 115 us, without the operand build 105, with a
-// quarter of the folds 99 (graph replay).
+// 2304 28.8 -> 25.6. The matrix pipe is busy 36% of the clocks, with a VALU op beside it in 63% of
+// those (27% with each sub-block's folds after its MFMAs). Timing-only copies (graph replay): without its
+// loads 109 of 115 us, without the operand build 105, with a quarter of the folds 99.
 //
 // Activation layout ("act32", k_act32_from_p32 from per-32 rows), for M_pad = m
 // rounded up to the workgroup's 32 TT rows (zero rows past m), T = M_pad / 32 row

@@ -228,7 +228,8 @@ DQ_API int dq_gemm(const dq_weight* w, int fmt, const void* acts, int64_t m, int
  * a row; under stream capture they take the one that needs no memory), while their GEMM adds the
  * blocks in another order. Replaces Device::matmul
  * (dynacore/include/dynacore/device/device.h:161; CpuDevice::matmul,
- * dynacore/cpu/cpu_device.cpp:869-1177). Uses a per-device scratch buffer. */
+ * dynacore/cpu/cpu_device.cpp:869-1177). Uses a per-device scratch buffer, or the stream's own
+ * (4..12 rows of Q8_0 / Q4_0). */
 DQ_API int dq_matmul(const dq_weight* w, const float* x, int64_t m, int64_t x_stride, float* y, int64_t y_stride,
                      const float* bias, void* stream);
 
@@ -273,7 +274,8 @@ typedef struct dq_matmul_job {
 
 /* Several independent matmuls on one stream, e.g. the projections that share one
  * input (Q/K/V, gate/up) or the experts of an MoE layer. One-row K-quant jobs of one k run
- * in one launch for up to 8 of them (weights of no more 64-row groups than CUs). The decode-sized K-quant
+ * in one launch for up to 8 of them (weights of no more 64-row groups than CUs, where that is
+ * faster). The decode-sized K-quant
  * jobs (Q4_K: 2 <= m <= 16; Q6_K: 2 <= m <= 64) of one k run together in grouped
  * skinny-GEMV launches (up to
  * 8 jobs each, Q4_K and Q6_K mixed) that quantize each job's fp32 rows in the
