@@ -23,13 +23,14 @@
 //
 // Work split: a workgroup owns 16 TC weight rows and all of K; TC = 4 (the weight load
 // instructions read 1 KB runs, the activations are prepared once per 64 weight rows) where
-// narrower ones would need a second round on the CUs, else 2 or 1 (N = 11008 Q8_0 at 8 rows 12.4 us
+// narrower ones would need a second round on the CUs, else 2 or 1 (N = 11008 Q8_0 at 8 rows 12.2 us
 // against 15.8 with 32-row workgroups). A wave's slices are contiguous in K. Of two short slices
 // (16 of a whole row) each takes two lane groups, which leaves no lane group idle at a slice's end;
-// one after the other they took 4.1 us instead of 3.3 at K = 1024, N = 4096. The long rows of
-// few row groups (two ranges and more) go slice by slice: a load of four consecutive blocks
-// touches half the cache lines of four slices' (Q8_0 K = 14336, N = 5120 at 8 rows 30.3 us
-// against 34.2), on 16 waves where one workgroup fills a CU (N = 2048, Q4_0 14.6 against 16.6).
+// one after the other they took 3.9 us instead of 3.0 at K = 1024, N = 4096. Slice by slice go the
+// long rows of few row groups (two ranges and more) and Q8_0's slices of 12 blocks and more: a load
+// of four consecutive blocks touches half the cache lines of four slices' (Q8_0 K = 14336, N = 5120
+// at 8 rows 30.3 us against 34.2; K = 7360, N = 14336 at 12 rows 22.2 against 24.1), on 16 waves
+// where one workgroup fills a CU (N = 2048, Q4_0 14.6 against 16.6).
 // What bounds it: Q4_0 K = 4096, N = 14336 at 8 rows takes 10.8 us for 33 MB (3.1 TB/s; the
 // VALU GEMV, which pays its dots for every row, 15.3). A wave's four steps are 44 MFMAs (768 clocks)
 // and ~350 VALU (1,400) each; loads one or two steps ahead measured alike.
@@ -244,6 +245,13 @@ hipError_t launch_type(const WeightDev& w, const uint8_t* acts, int64_t stride, 
   switch (gemv_splits(w, kActPer32)) {
     case 1:
       if (gemv_waves32(w, kActPer32) == 8) return DQ_ROWS32(4, 8, 1, 8, 1);
+      if constexpr (WT == kQ8_0) {
+        // long slices one after the other where that takes (nearly) no more steps
+        const int64_t slice = (w.nblk + 15) / 16;
+        if (slice >= 20 || (slice >= 12 && (slice + 1) % 4 <= 1)) {
+          return tc == 4 ? DQ_ROWS32(4, 8, 1, 16, 1) : tc == 2 ? DQ_ROWS32(2, 8, 1, 16, 1) : DQ_ROWS32(1, 8, 1, 16, 1);
+        }
+      }
       return tc == 4 ? DQ_ROWS32(4, 8, 1, 16, 2) : tc == 2 ? DQ_ROWS32(2, 8, 1, 16, 2) : DQ_ROWS32(1, 8, 1, 16, 2);
     case 2: return tc == 1 ? DQ_ROWS32(1, 8, 2, 8, 1) : DQ_ROWS32(2, 8, 2, 8, 1);
     case 3: return DQ_ROWS32(1, 8, 3, 8, 1);

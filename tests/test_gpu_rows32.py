@@ -117,7 +117,8 @@ def test_infinite_last_block(cuda, t, k):
 # than CUs), two to eight ranges of 8 -- with slices of no, a few and uneven blocks
 @pytest.mark.parametrize("t", TYPES32, ids=lambda t: O.TYPE_NAMES[t])
 @pytest.mark.parametrize("n,k", [(70, 32), (300, 1504), (6200, 416), (14336, 96), (16500, 160), (6000, 8192), (7000, 8224),
-                                 (5000, 8192), (4096, 8288), (3100, 8192), (2600, 8224), (2304, 8192), (130, 14336)])
+                                 (5000, 8192), (4096, 8288), (3100, 8192), (2600, 8224), (2304, 8192), (130, 14336),
+                                 (200, 7360), (6200, 6144), (9000, 11008)])
 def test_the_one_row_bits(cuda, t, n, k):
     """A row's outputs are the one-row call's bit for bit whatever the rows beside it, from fp32 rows
     and from quantized ones, and for rows whose scales and products fall below the normal range."""
