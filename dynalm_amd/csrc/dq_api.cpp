@@ -149,12 +149,22 @@ struct StreamWs {
 std::mutex g_sws_mu;
 std::vector<StreamWs> g_sws;
 
-// This thread's stream-capture mode is "relaxed" for the object's life: an allocation neither fails
-// for nor invalidates a capture that another thread has begun.
+// Whether the stream is not capturing: a captured launch keeps its buffers' addresses, and a
+// later call may grow (free) the stream's workspace, so a route that can do without one does
+// under capture.
+bool not_capturing(void* stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(as_stream(stream), &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // not this call's error: the launches after it report their own
+  return false;
+}
+
+// This thread's stream-capture mode is "relaxed" for the object's life (if `on`): an allocation
+// neither fails for nor invalidates a capture that another thread has begun.
 struct RelaxedCapture {
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   bool ok;
-  RelaxedCapture() : ok(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+  explicit RelaxedCapture(bool on) : ok(on && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
   ~RelaxedCapture() {
     if (ok) (void)hipThreadExchangeStreamCaptureMode(&mode);  // (back to what it was)
   }
@@ -174,7 +184,7 @@ hipError_t stream_ws(int device, void* stream, size_t need, uint8_t** out, const
     dq::DeviceScope ds(device);
     *what = "hipSetDevice";
     if (ds.err != hipSuccess) return ds.err;
-    RelaxedCapture relaxed;
+    RelaxedCapture relaxed(not_capturing(stream));  // (under its own capture the allocation is refused)
     hipError_t rc = hipSuccess;
     if (e->p != nullptr) {
       *what = "hipStreamSynchronize";
@@ -203,16 +213,6 @@ int with_stream_ws(int device, void* stream, size_t need, F&& fn) {
   const char* what = "";
   DQ_HIP(stream_ws(device, stream, need, &p, &what), what);
   return fn(p);
-}
-
-// Whether the stream is not capturing: a captured launch keeps its buffers' addresses, and a
-// later call may grow (free) the stream's workspace, so a route that can do without one does
-// under capture.
-bool not_capturing(void* stream) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(as_stream(stream), &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
-  (void)hipGetLastError();  // not this call's error: the launches after it report their own
-  return false;
 }
 
 // The quantized-activation buffer of one matmul: the start of the caller's region,

@@ -108,6 +108,12 @@ assert count(w, 8) == 2 and var("relaxed_mallocs").value == before + 1
 m = ctypes.c_int(0)
 fake.hipThreadExchangeStreamCaptureMode(ctypes.byref(m))
 assert m.value == 0
+# a stream that captures itself keeps the mode that refuses: its graph would outlive the buffer
+wk = weight(dq.Q4_K, 300, 512)
+before = var("relaxed_mallocs").value
+var("capturing").value = 1
+dq.gemm(wk, dq.ACT_PER32, 64, 64, 0, wk.n, 64, wk.n, None, 0x2000)
+assert var("relaxed_mallocs").value == before
 """)
 
 
